@@ -6,10 +6,9 @@
 // (nh); the steps' workspace spectrum uses pitch = nh.
 //
 // Transforms are mixed-radix Stockham (self-sorting, decimation in time)
-// passes on lines staged in LDS.  A workgroup owns `lpw` lines laid out
-// element-major (LDS index e*lpw + line) and `tpl` threads per line; thread
-// `tid` works on line tid % lpw.  Radices 2, 3, 4, 5 and 8 have closed-form
-// butterflies; any other prime factor up to 31 uses a generic O(R^2) DFT.
+// passes: size-specialised kernels (evx_fft_tiles.hpp) where one exists, the
+// runtime-radix line kernels (evx_fft_lines.hpp) for every other length with
+// prime factors up to 31.
 //
 // Sweeps of one IMEX step (each reads and writes HBM once):
 //   z : RHS lines (pairs packed as one complex line) -> half spectra
@@ -24,6 +23,7 @@
 
 #include "evx_common.hpp"
 #include "evx_fft_engine.hpp"
+#include "evx_fft_lines.hpp"
 #include "evx_fft_tiles.hpp"
 #include "evx_rz_tile.hpp"
 
@@ -42,240 +42,7 @@ int stencil_rhs_rd_periodic(int32_t dtype, const void* u, void* out, const Dims&
 
 namespace {
 
-constexpr int MAXPASS = 24;
-constexpr int EMAX = 32;           // max complex values a thread holds in one pass
 constexpr size_t LDS_BUDGET = 64 * 1024;
-
-template <typename T>
-struct Axis {
-  int n;
-  int npass;
-  int tpl;
-  int radix[MAXPASS];
-  const cpx<T>* tw;  // n roots of unity exp(-2 pi i m / n)
-};
-
-// One Stockham pass of radix R over every line of the workgroup.
-// p = product of the radices already applied.  Butterfly i (0 <= i < n/R)
-// reads elements i + r*n/R, twiddles by w_{pR}^{r*(i mod p)}, and writes
-// (i - i mod p)*R + i mod p + r*p.
-template <typename T, bool INV, int R>
-__device__ __forceinline__ void pass_fixed(cpx<T>* buf, int lpw, int line, int tl, int tpl, int n, int p,
-                                           const cpx<T>* tw, bool active) {
-  constexpr int SMAX = EMAX / R;
-  const int m = n / R;
-  const int stride = n / (p * R);
-  cpx<T> y[SMAX][R];
-#pragma unroll
-  for (int s = 0; s < SMAX; ++s) {
-    const int i = tl + s * tpl;
-    if (active && i < m) {
-      const int k = i % p;
-      cpx<T> x[R];
-#pragma unroll
-      for (int r = 0; r < R; ++r) x[r] = buf[(i + r * m) * lpw + line];
-      if (p > 1) {
-#pragma unroll
-        for (int r = 1; r < R; ++r) {
-          const cpx<T> w = tw[r * k * stride];
-          x[r] = INV ? cmulc(x[r], w) : cmul(x[r], w);
-        }
-      }
-      dft_fixed<T, INV, R>(x);
-#pragma unroll
-      for (int r = 0; r < R; ++r) y[s][r] = x[r];
-    }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int s = 0; s < SMAX; ++s) {
-    const int i = tl + s * tpl;
-    if (active && i < m) {
-      const int k = i % p;
-      const int j = (i - k) * R + k;
-#pragma unroll
-      for (int r = 0; r < R; ++r) buf[(j + r * p) * lpw + line] = y[s][r];
-    }
-  }
-  __syncthreads();
-}
-
-// Generic odd-prime radix: y_q = sum_r (x_r w^{rk}) w_R^{rq}, O(R^2).
-template <typename T, bool INV>
-__device__ __noinline__ void pass_generic(cpx<T>* buf, int lpw, int line, int tl, int tpl, int n, int p, int R,
-                                          const cpx<T>* tw, bool active) {
-  const int m = n / R;
-  const int stride = n / (p * R);
-  const int nr = n / R;
-  cpx<T> y[EMAX];
-  int cnt = 0;
-  for (int i = tl; active && i < m; i += tpl) {
-    const int k = i % p;
-    for (int q = 0; q < R; ++q) {
-      cpx<T> acc = {T(0), T(0)};
-      for (int r = 0; r < R; ++r) {
-        cpx<T> xr = buf[(i + r * m) * lpw + line];
-        const cpx<T> w = tw[r * k * stride];
-        xr = INV ? cmulc(xr, w) : cmul(xr, w);
-        const cpx<T> wq = tw[((r * q) % R) * nr];
-        acc = cadd(acc, INV ? cmulc(xr, wq) : cmul(xr, wq));
-      }
-      y[cnt++] = acc;
-    }
-  }
-  __syncthreads();
-  cnt = 0;
-  for (int i = tl; active && i < m; i += tpl) {
-    const int k = i % p;
-    const int j = (i - k) * R + k;
-    for (int q = 0; q < R; ++q) buf[(j + q * p) * lpw + line] = y[cnt++];
-  }
-  __syncthreads();
-}
-
-template <typename T, bool INV>
-__device__ void fft_lines(cpx<T>* buf, int lpw, int line, int tl, const Axis<T>& a, const cpx<T>* tw,
-                          bool active) {
-  int p = 1;
-  for (int s = 0; s < a.npass; ++s) {
-    const int R = a.radix[s];
-    switch (R) {
-      case 8: pass_fixed<T, INV, 8>(buf, lpw, line, tl, a.tpl, a.n, p, tw, active); break;
-      case 4: pass_fixed<T, INV, 4>(buf, lpw, line, tl, a.tpl, a.n, p, tw, active); break;
-      case 2: pass_fixed<T, INV, 2>(buf, lpw, line, tl, a.tpl, a.n, p, tw, active); break;
-      case 3: pass_fixed<T, INV, 3>(buf, lpw, line, tl, a.tpl, a.n, p, tw, active); break;
-      case 5: pass_fixed<T, INV, 5>(buf, lpw, line, tl, a.tpl, a.n, p, tw, active); break;
-      default: pass_generic<T, INV>(buf, lpw, line, tl, a.tpl, a.n, p, R, tw, active); break;
-    }
-    p *= R;
-  }
-}
-
-template <typename T>
-__device__ __forceinline__ void load_twiddles(cpx<T>* tw, const Axis<T>& a) {
-  for (int i = threadIdx.x; i < a.n; i += blockDim.x) tw[i] = a.tw[i];
-}
-
-// --------------------------------------------------------------- z sweeps --
-// Real lines of length n along z; line pairs (2q, 2q+1) form one complex line.
-template <typename T>
-__global__ void z_r2c_kernel(const T* __restrict__ x, cpx<T>* __restrict__ spec, int64_t nlines, int nh,
-                             int64_t pitch, Axis<T> a, int lpw) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  cpx<T>* tw = reinterpret_cast<cpx<T>*>(smem_raw);
-  cpx<T>* buf = tw + a.n;
-  const int n = a.n, tid = threadIdx.x;
-  load_twiddles(tw, a);
-  const int64_t l0 = (int64_t)blockIdx.x * lpw * 2;
-  const int nl = (int)min((int64_t)2 * lpw, nlines - l0);
-  const int np = (nl + 1) / 2;
-  const T* src = x + l0 * n;
-  for (int q = tid; q < 2 * np * n; q += blockDim.x) {
-    const int l = q / n, e = q - (q / n) * n;
-    const T v = l < nl ? src[q] : T(0);
-    T* z = reinterpret_cast<T*>(&buf[e * lpw + (l >> 1)]);
-    z[l & 1] = v;
-  }
-  __syncthreads();
-  const int line = tid % lpw, tl = tid / lpw;
-  fft_lines<T, false>(buf, lpw, line, tl, a, tw, line < np && tl < a.tpl);
-  cpx<T>* dst = spec + l0 * pitch;
-  for (int q = tid; q < nl * nh; q += blockDim.x) {
-    const int l = q / nh, k = q - (q / nh) * nh;
-    const cpx<T> Z = buf[k * lpw + (l >> 1)];
-    const cpx<T> Zc = buf[((n - k) % n) * lpw + (l >> 1)];
-    cpx<T> o;
-    if ((l & 1) == 0) o = {(Z.x + Zc.x) * T(0.5), (Z.y - Zc.y) * T(0.5)};
-    else o = {(Z.y + Zc.y) * T(0.5), (Zc.x - Z.x) * T(0.5)};
-    dst[l * pitch + k] = o;
-  }
-}
-
-template <typename T>
-__device__ __forceinline__ cpx<T> herm_load(const cpx<T>* line, int k, int n, int nh) {
-  cpx<T> v = k < nh ? line[k] : cpx<T>{line[n - k].x, -line[n - k].y};
-  if (k == 0 || 2 * k == n) v.y = T(0);  // C2R ignores Im of the DC and Nyquist bins
-  return v;
-}
-
-// out = base + scale * irfft(spec) per line (base may be NULL; out may alias base).
-template <typename T>
-__global__ void z_c2r_kernel(const cpx<T>* __restrict__ spec, T* out, const T* base, T scale, int64_t nlines,
-                             int nh, int64_t pitch, Axis<T> a, int lpw) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  cpx<T>* tw = reinterpret_cast<cpx<T>*>(smem_raw);
-  cpx<T>* buf = tw + a.n;
-  const int n = a.n, tid = threadIdx.x;
-  load_twiddles(tw, a);
-  const int64_t l0 = (int64_t)blockIdx.x * lpw * 2;
-  const int nl = (int)min((int64_t)2 * lpw, nlines - l0);
-  const int np = (nl + 1) / 2;
-  for (int q = tid; q < np * n; q += blockDim.x) {
-    const int pr = q / n, k = q - (q / n) * n;
-    const cpx<T>* la = spec + (l0 + 2 * pr) * pitch;
-    const cpx<T> A = herm_load(la, k, n, nh);
-    const cpx<T> B = (2 * pr + 1 < nl) ? herm_load(la + pitch, k, n, nh) : cpx<T>{T(0), T(0)};
-    buf[k * lpw + pr] = {A.x - B.y, A.y + B.x};
-  }
-  __syncthreads();
-  const int line = tid % lpw, tl = tid / lpw;
-  fft_lines<T, true>(buf, lpw, line, tl, a, tw, line < np && tl < a.tpl);
-  T* o = out + l0 * n;
-  const T* b = base ? base + l0 * n : nullptr;
-  for (int q = tid; q < nl * n; q += blockDim.x) {
-    const int l = q / n, e = q - (q / n) * n;
-    const T* z = reinterpret_cast<const T*>(&buf[e * lpw + (l >> 1)]);
-    const T v = scale * z[l & 1];
-    o[q] = b ? b[q] + v : v;
-  }
-}
-
-
-// MODE 0: forward, 1: inverse, 2/3: forward * prefac * inverse (x axis only;
-// 3 with the exact-symbol multiplier)
-template <typename T, int MODE>
-__global__ void strided_kernel(cpx<T>* spec, int64_t nlines, LineMap lm, Axis<T> a, int lpw, Prefac pf) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  cpx<T>* tw = reinterpret_cast<cpx<T>*>(smem_raw);
-  cpx<T>* buf = tw + a.n;
-  const int n = a.n, tid = threadIdx.x;
-  load_twiddles(tw, a);
-  const int64_t L0 = (int64_t)blockIdx.x * lpw;
-  const int nl = (int)min((int64_t)lpw, nlines - L0);
-  // blockDim.x is a multiple of lpw, so each thread always serves line tid % lpw.
-  const int line = tid % lpw, tl = tid / lpw, jstep = blockDim.x / lpw;
-  const int64_t start = line < nl ? line_start(lm, L0 + line) : 0;
-  if (line < nl)
-    for (int j = tl; j < n; j += jstep) buf[j * lpw + line] = spec[start + j * lm.es];
-  __syncthreads();
-  const bool active = line < nl && tl < a.tpl;
-  if (MODE == 1) {
-    fft_lines<T, true>(buf, lpw, line, tl, a, tw, active);
-  } else {
-    fft_lines<T, false>(buf, lpw, line, tl, a, tw, active);
-  }
-  if (MODE >= 2) {
-    const T sc = static_cast<T>(pf.scale);
-    if (line < nl) {
-      const int64_t L = L0 + line;
-      const int64_t outer = L / lm.nh;
-      const int jz = (int)(L - outer * lm.nh);
-      const int jy = (int)(outer % pf.ny);
-      const float ssc = symbol_scalar(pf, outer / pf.ny);
-      for (int j = tl; j < n; j += jstep) {
-        const T f = pf.etd     ? static_cast<T>(etd1_f32(j, jy, jz, pf, ssc)) * sc
-                    : pf.exact ? static_cast<T>(prefac_f64(j, jy, jz, pf, outer / pf.ny) * pf.scale)
-                               : static_cast<T>(prefac_f32(j, jy, jz, pf, ssc)) * sc;
-        buf[j * lpw + line] = cscale(buf[j * lpw + line], f);
-      }
-    }
-    __syncthreads();
-    fft_lines<T, true>(buf, lpw, line, tl, a, tw, active);
-  }
-  if (line < nl)
-    for (int j = tl; j < n; j += jstep) spec[start + j * lm.es] = buf[j * lpw + line];
-}
-
 
 template <typename T, int N>
 __global__ __launch_bounds__((ZGeo<T, N>::THREADS)) void z_r2c_fast(const T* __restrict__ x, cpx<T>* __restrict__ spec,
@@ -337,18 +104,6 @@ int64_t x_pipe_resident() {
     return (int64_t)per * cus;
   }();
   return resident;
-}
-
-// Sizes with size-specialised kernels.
-bool fast_size(int n) {
-  switch (n) {
-#define X(NN) case NN:
-    EVX_FAST_SIZES(X)
-#undef X
-    return true;
-    default:
-      return false;
-  }
 }
 
 template <typename T>
@@ -435,38 +190,11 @@ std::vector<int> factorize(int n) {
   return r;
 }
 
-// Threads per line such that no pass needs more than EMAX values per thread.
-int min_tpl(int n, const std::vector<int>& rad) {
-  int tpl = 1;
-  for (;;) {
-    bool ok = true;
-    for (int R : rad) {
-      const int m = n / R;
-      if (((m + tpl - 1) / tpl) * R > EMAX) { ok = false; break; }
-    }
-    if (ok) return tpl;
-    ++tpl;
-  }
-}
-
-// Largest threads-per-line <= tmax for which every pass is balanced (each
-// thread gets the same butterfly count); tpl_min if none is.
-int pick_tpl(int n, const std::vector<int>& rad, int tpl_min, int tmax) {
-  if (rad.empty()) return 1;
-  for (int t = tmax; t >= tpl_min; --t) {
-    bool ok = true;
-    for (int R : rad)
-      if ((n / R) % t) { ok = false; break; }
-    if (ok) return t;
-  }
-  return tpl_min;
-}
-
 struct AxisHost {
   int n = 1;
-  std::vector<int> rad;
-  int tpl_min = 1;
-  void* tw = nullptr;  // device
+  LinePlan line;         // passes of the runtime-radix kernels
+  void* tw = nullptr;    // in the plan's tables: n roots of unity (size-specialised kernels)
+  void* ltab = nullptr;  // in the plan's tables: the table of `line`
 };
 
 }  // namespace
@@ -478,6 +206,7 @@ struct evx_fft_plan {
   int64_t nh;
   int64_t pitch;  // row pitch (complex values) of the workspace spectrum, >= nh
   evx::AxisHost ax[3];  // x, y, z (z: complex length nz)
+  void* tables = nullptr;  // device buffer of the axes' tables
   // One-shot stage trace: events recorded around the kernels of the next step.
   // One-shot launch trace of the next step: event 0 before the first kernel,
   // event i after the i-th kernel, whose kind is kinds[i-1].
@@ -495,73 +224,35 @@ struct evx_fft_plan {
 namespace evx {
 namespace {
 
+// The tables of all three axes in one device buffer (one allocation, one
+// upload): the first step on a new grid shape pays for them.
 template <typename T>
-Axis<T> axis_dev(const AxisHost& h, int tpl) {
-  Axis<T> a;
-  a.n = h.n;
-  a.npass = (int)h.rad.size();
-  for (int i = 0; i < a.npass; ++i) a.radix[i] = h.rad[i];
-  a.tpl = tpl;
-  a.tw = static_cast<const cpx<T>*>(h.tw);
-  return a;
-}
-
-template <typename T>
-int make_twiddles(AxisHost& h) {
-  std::vector<cpx<T>> t(h.n);
+int make_twiddles(AxisHost (&ax)[3], void** buf) {
   const long double tau = 6.283185307179586476925286766559005768L;
-  for (int m = 0; m < h.n; ++m) {
-    const long double ang = tau * (long double)m / (long double)h.n;
-    t[m].x = static_cast<T>(cosl(ang));
-    t[m].y = static_cast<T>(-sinl(ang));
+  auto root = [&](int64_t j, int64_t n) {
+    const long double ang = tau * (long double)(j % n) / (long double)n;
+    return cpx<T>{static_cast<T>(cosl(ang)), static_cast<T>(-sinl(ang))};
+  };
+  auto aligned = [](size_t n) { return (n + 15) & ~size_t(15); };
+  size_t total = 0;
+  for (const AxisHost& h : ax) total += aligned(h.n) + aligned(h.line.tab);
+  std::vector<cpx<T>> t(total);
+  if (hipMalloc(buf, sizeof(cpx<T>) * total) != hipSuccess) {
+    *buf = nullptr;
+    return fail(EVX_ERR_NOMEM, "hipMalloc of %zu twiddles failed", total);
   }
-  if (hipMalloc(&h.tw, sizeof(cpx<T>) * h.n) != hipSuccess) {
-    h.tw = nullptr;
-    return fail(EVX_ERR_NOMEM, "hipMalloc of %d twiddles failed", h.n);
+  size_t at = 0;
+  for (AxisHost& h : ax) {
+    for (int m = 0; m < h.n; ++m) t[at + m] = root(m, h.n);
+    h.tw = static_cast<cpx<T>*>(*buf) + at;
+    at += aligned(h.n);
+    line_fill_table(h.line, t.data() + at, root);
+    h.ltab = static_cast<cpx<T>*>(*buf) + at;
+    at += aligned(h.line.tab);
   }
-  if (hipMemcpy(h.tw, t.data(), sizeof(cpx<T>) * h.n, hipMemcpyHostToDevice) != hipSuccess)
+  if (hipMemcpy(*buf, t.data(), sizeof(cpx<T>) * total, hipMemcpyHostToDevice) != hipSuccess)
     return fail(EVX_ERR_HIP, "twiddle upload failed");
   return EVX_OK;
-}
-
-// Launch geometry: lines per workgroup and threads per line for an axis.
-struct Geom {
-  int lpw, tpl, threads;
-  size_t lds;
-};
-
-template <typename T>
-Geom z_geom(const AxisHost& h, int64_t npairs) {
-  Geom g;
-  g.tpl = pick_tpl(h.n, h.rad, h.tpl_min, 64);
-  // Prefer ~256 threads per workgroup within the LDS budget.
-  const size_t line_bytes = sizeof(cpx<T>) * h.n;
-  int lpw = 256 / g.tpl;
-  if (lpw < 1) lpw = 1;
-  while (lpw > 1 && line_bytes * (lpw + 1) > LDS_BUDGET) --lpw;
-  if (lpw > npairs) lpw = (int)(npairs < 1 ? 1 : npairs);
-  g.lpw = lpw;
-  g.threads = lpw * g.tpl;
-  if (g.threads > 1024) g.threads = 1024;
-  g.lds = line_bytes * (lpw + 1);
-  return g;
-}
-
-template <typename T>
-Geom strided_geom(const AxisHost& h, int64_t nlines) {
-  Geom g;
-  g.tpl = pick_tpl(h.n, h.rad, h.tpl_min, 16);
-  const size_t line_bytes = sizeof(cpx<T>) * h.n;
-  int lpw = 16;  // 16 adjacent lines: 128 B (f32) / 256 B (f64) contiguous runs
-  if (lpw * g.tpl > 1024) lpw = 1024 / g.tpl;
-  if (lpw < 1) lpw = 1;
-  while (lpw * g.tpl < 256 && line_bytes * (2 * lpw + 1) <= LDS_BUDGET && 2 * lpw * g.tpl <= 1024) lpw *= 2;
-  while (lpw > 1 && line_bytes * (lpw + 1) > LDS_BUDGET) --lpw;
-  if (lpw > nlines) lpw = (int)(nlines < 1 ? 1 : nlines);
-  g.lpw = lpw;
-  g.threads = lpw * g.tpl;
-  g.lds = line_bytes * (lpw + 1);
-  return g;
 }
 
 template <typename T>
@@ -577,11 +268,7 @@ int run_z_r2c(evx_fft_plan* p, const void* x, void* spec, int64_t pitch, hipStre
     nlines = (xb - xa) * p->d.ny;
   }
   if (p->fast && fast_z_r2c<T>(h.n, x, spec, nlines, pitch, h.tw, s)) return check_launch("z_r2c_fast");
-  const Geom g = z_geom<T>(h, (nlines + 1) / 2);
-  const int64_t blocks = (nlines + 2 * g.lpw - 1) / (2 * g.lpw);
-  hipLaunchKernelGGL(z_r2c_kernel<T>, dim3((unsigned)blocks), dim3(g.threads), g.lds, s, static_cast<const T*>(x),
-                     static_cast<cpx<T>*>(spec), nlines, (int)p->nh, pitch, axis_dev<T>(h, g.tpl), g.lpw);
-  return check_launch("z_r2c_kernel");
+  return line_run_z_r2c<T>(h.line, h.ltab, x, spec, nlines, pitch, s);
 }
 
 template <typename T>
@@ -599,15 +286,10 @@ int run_z_c2r(evx_fft_plan* p, const void* spec, void* out, const void* base, do
   if (p->fast && fast_z_c2r<T>(h.n, spec, out, base, scale, nlines, pitch, h.tw, s, rec))
     return check_launch("z_c2r_fast");
   if (rec) return fail(EVX_ERR_INVALID, "step sums need the size-specialised z C2R");
-  const Geom g = z_geom<T>(h, (nlines + 1) / 2);
-  const int64_t blocks = (nlines + 2 * g.lpw - 1) / (2 * g.lpw);
-  hipLaunchKernelGGL(z_c2r_kernel<T>, dim3((unsigned)blocks), dim3(g.threads), g.lds, s,
-                     static_cast<const cpx<T>*>(spec), static_cast<T*>(out), static_cast<const T*>(base),
-                     static_cast<T>(scale), nlines, (int)p->nh, pitch, axis_dev<T>(h, g.tpl), g.lpw);
-  return check_launch("z_c2r_kernel");
+  return line_run_z_c2r<T>(h.line, h.ltab, spec, out, base, scale, nlines, pitch, s);
 }
 
-// mirror (x sweeps of the size-specialised kernels only): see LineMap.
+// mirror (x sweeps): see LineMap.
 template <typename T, int MODE>
 int run_strided(evx_fft_plan* p, int axis, void* spec, const Prefac& pf, int64_t pitch, hipStream_t s,
                 int64_t xa = 0, int64_t xb = -1, int mirror = 0) {
@@ -636,12 +318,8 @@ int run_strided(evx_fft_plan* p, int axis, void* spec, const Prefac& pf, int64_t
   }
   if (h.n == 1 && MODE < 2) return EVX_OK;  // length-1 transform is the identity
   if (p->fast && fast_strided<T, MODE>(h.n, spec, nlines, lm, h.tw, pf, s)) return check_launch("strided_fast");
-  if (mirror) return fail(EVX_ERR_UNSUPPORTED, "mirrored sweeps need a size-specialised transform");
-  const Geom g = strided_geom<T>(h, nlines);
-  const int64_t blocks = (nlines + g.lpw - 1) / g.lpw;
-  hipLaunchKernelGGL((strided_kernel<T, MODE>), dim3((unsigned)blocks), dim3(g.threads), g.lds, s,
-                     static_cast<cpx<T>*>(spec), nlines, lm, axis_dev<T>(h, g.tpl), g.lpw, pf);
-  return check_launch("strided_kernel");
+  // the runtime-radix kernel takes the kind of multiplier from pf
+  return line_run_strided<T>(MODE < 2 ? MODE : 2, h.line, h.ltab, spec, nlines, lm, pf, s);
 }
 
 Prefac make_prefac(const evx_fft_plan* p, int ch, double sym_scalar, double dt, const double spacing[3]) {
@@ -928,32 +606,25 @@ extern "C" int evx_fft_plan_create(evx_fft_plan** out, int32_t dtype, int64_t ch
   for (int a = 0; a < 3; ++a) {
     AxisHost& h = p->ax[a];
     h.n = (int)n[a];
-    h.rad = factorize(h.n);
-    if (h.n == 1) h.rad.clear();
-    for (int R : h.rad)
+    for (int R : factorize(h.n))
       if (R > 31) {
         evx_fft_plan_destroy(p);
         return fail(EVX_ERR_UNSUPPORTED, "axis length %d has a prime factor %d > 31", h.n, R);
       }
-    if ((int)h.rad.size() > MAXPASS) {
-      evx_fft_plan_destroy(p);
-      return fail(EVX_ERR_UNSUPPORTED, "axis length %d needs too many passes", h.n);
-    }
-    h.tpl_min = min_tpl(h.n, h.rad);
-    if (h.tpl_min > 1024) {
-      evx_fft_plan_destroy(p);
-      return fail(EVX_ERR_UNSUPPORTED, "axis length %d needs more than 1024 threads per line", h.n);
-    }
     const size_t elem = dtype == EVX_F32 ? sizeof(cpx<float>) : sizeof(cpx<double>);
     if (elem * h.n * 2 > LDS_BUDGET) {
       evx_fft_plan_destroy(p);
       return fail(EVX_ERR_UNSUPPORTED, "axis length %d exceeds the LDS line budget", h.n);
     }
-    const int st = dtype == EVX_F32 ? make_twiddles<float>(h) : make_twiddles<double>(h);
-    if (st != EVX_OK) {
+    if (!line_make_plan(h.n, dtype == EVX_F64, &h.line)) {
       evx_fft_plan_destroy(p);
-      return st;
+      return fail(EVX_ERR_UNSUPPORTED, "axis length %d needs too many passes", h.n);
     }
+  }
+  const int st = dtype == EVX_F32 ? make_twiddles<float>(p->ax, &p->tables) : make_twiddles<double>(p->ax, &p->tables);
+  if (st != EVX_OK) {
+    evx_fft_plan_destroy(p);
+    return st;
   }
   *out = p;
   return EVX_OK;
@@ -961,8 +632,7 @@ extern "C" int evx_fft_plan_create(evx_fft_plan** out, int32_t dtype, int64_t ch
 
 extern "C" int evx_fft_plan_destroy(evx_fft_plan* p) {
   if (!p) return EVX_OK;
-  for (auto& h : p->ax)
-    if (h.tw) (void)hipFree(h.tw);
+  if (p->tables) (void)hipFree(p->tables);
   delete p;
   return EVX_OK;
 }
@@ -1136,10 +806,10 @@ int mirror_spectral_step(evx_fft_plan* p, int ch, const void* u, void* u_out, vo
              : evx_rd_rhs(p->dtype, u, rhs, &g, bc, prm->D, &e, s));
   EVX_TRY(trace_tick(p, TK_RHS, s));
   const int mode = staggered ? 2 : (dir ? 1 : 0);
-  // Cell-centred extensions (N = 2n) on a size-specialised x transform: the
-  // x sweep reads the upper half as the mirror image of the lower half and
-  // stores the lower half only; otherwise the half spectrum is extended first.
-  const bool xmir = !staggered && p->fast && fast_size((int)NX);
+  // Cell-centred extensions (N = 2n): the x sweep reads the upper half as the
+  // mirror image of the lower half and stores the lower half only; staggered
+  // ones extend the half spectrum first.
+  const bool xmir = !staggered;
   const int xmode = xmir ? (dir ? 2 : 1) : 0;
   const int64_t ext = staggered ? n + 2 : n;  // extension planes
   const int64_t cplane = p->d.ny * p->pitch;   // complex elements per spectrum plane

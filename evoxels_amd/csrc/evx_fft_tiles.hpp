@@ -24,11 +24,6 @@ struct LineMap {
   int32_t mirror = 0;
 };
 
-__device__ __forceinline__ int64_t line_start(const LineMap& m, int64_t L) {
-  const int64_t outer = L / m.nh, k = L - (L / m.nh) * m.nh;
-  return (outer / m.G) * m.GM + (outer % m.G) * m.OM + k;
-}
-
 // Line L0 + t of a brick whose first line L0 is block-uniform: the divisions
 // resolve L0 once per wave; a lane's line carries k into o and o into g
 // (k = L % nh, o = outer % G, g = outer / G, outer = L / nh), which takes a

@@ -36,6 +36,8 @@ constexpr int BT = 256;  // threads of every batched workgroup
 // FFT sizes the batched kernels are built for (all give 256-thread tiles).
 #define EVX_BATCH_SIZES(X) X(16) X(32) X(48) X(64) X(96) X(128)
 
+using ChB = ChPer<float, 32, 2>;  // CH tiles: 16 x 32 points, the z lengths are 16 to 128
+
 constexpr size_t cmax(size_t a, size_t b) { return a > b ? a : b; }
 
 template <int N>
@@ -43,7 +45,7 @@ constexpr size_t fft_lds() {
   return cmax(ZTile<T, N>::LDS_BYTES, cmax(STile<T, N, 0>::LDS_BYTES, STile<T, N, 2>::LDS_BYTES));
 }
 constexpr size_t BATCH_LDS =
-    cmax(ChTile<T>::LDS_BYTES,
+    cmax(ChB::LDS_BYTES,
          cmax(fft_lds<16>(), cmax(fft_lds<32>(), cmax(fft_lds<48>(), cmax(fft_lds<64>(), cmax(fft_lds<96>(),
                                                                                            fft_lds<128>()))))));
 static_assert(BATCH_LDS <= 160 * 1024 / 3, "three batched workgroups must fit one CU's LDS");
@@ -130,10 +132,6 @@ __device__ __forceinline__ void strided_dispatch(const BInst& b, C* spec, const 
   }
 }
 
-// One item: it = {grid, sweep, first tile, tile count}.  GROUP = false:
-// items of one tile (the count is not read, and the tile loops vanish at
-// compile time); the grouped kernel is a separate instantiation, so its
-// register needs never touch the one-tile schedule.
 // Sweep ST of one item: it = {grid, sweep ST, first tile, tile count}.
 // GROUP = false: items of one tile (the count is not read, and the tile
 // loops vanish at compile time); the grouped kernels are separate
@@ -144,9 +142,8 @@ __device__ __forceinline__ void run_sweep(const BArgs& a, int4 it, int tid, unsi
   const int tile = it.z, count = GROUP ? it.w : 1;
   if constexpr (ST == 0) {
     const Dims d{1, b.nx, b.ny, b.nz};
-    Bc bc{};
-    const Epi ep{EVX_OUT_RHS, 0.0, nullptr, nullptr, nullptr};
-    ch_rhs_tile<T, false>(a.u + b.u_off, a.rhs + b.r_off, d, bc, b.g, b.k, ep, b.tg, nullptr, tile, tid, smem);
+    ch_periodic_tile<T, ChB::TZ, ChB::PY, false>(a.u + b.u_off, a.rhs + b.r_off, d, b.g, b.k, b.tg, nullptr, tile, tid,
+                                                 smem);
   } else if constexpr (ST == 1) {
     const int64_t nlines = (int64_t)b.nx * b.ny;
     switch (b.nz) {
@@ -181,23 +178,19 @@ __device__ __forceinline__ void run_sweep(const BArgs& a, int4 it, int tid, unsi
   }
 }
 
-// One item of any sweep.
-template <bool GROUP>
-__device__ __forceinline__ void run_item(const BArgs& a, int4 it, int tid, unsigned char* smem) {
-  switch (it.y) {
-    case 0: run_sweep<0, GROUP>(a, it, tid, smem); break;
-    case 1: run_sweep<1, GROUP>(a, it, tid, smem); break;
-    case 2: run_sweep<2, GROUP>(a, it, tid, smem); break;
-    case 3: run_sweep<3, GROUP>(a, it, tid, smem); break;
-    case 4: run_sweep<4, GROUP>(a, it, tid, smem); break;
-    default: run_sweep<5, GROUP>(a, it, tid, smem); break;
-  }
+// One sweep of every grid.  A kernel per sweep: each holds only its own
+// sweep's registers and LDS (one kernel for all six needed 97 registers and
+// 27 KB in every launch).
+template <int ST>
+constexpr size_t stage_lds() {
+  constexpr size_t z = cmax(cmax(cmax(ZTile<T, 16>::LDS_BYTES, ZTile<T, 32>::LDS_BYTES), cmax(ZTile<T, 48>::LDS_BYTES, ZTile<T, 64>::LDS_BYTES)), cmax(ZTile<T, 96>::LDS_BYTES, ZTile<T, 128>::LDS_BYTES));
+  return ST == 0 ? ChB::LDS_BYTES : ST == 1 || ST == 5 ? z : BATCH_LDS;
 }
 
-template <bool GROUP>
-__global__ __launch_bounds__(BT) void batch_stage(BArgs a, int first) {
-  __shared__ __align__(16) unsigned char smem[BATCH_LDS];
-  run_item<GROUP>(a, a.items[first + (int)blockIdx.x], threadIdx.x, smem);
+template <int ST, bool GROUP>
+__global__ __launch_bounds__(BT) void batch_stage(BArgs a) {
+  __shared__ __align__(16) unsigned char smem[stage_lds<ST>()];
+  run_sweep<ST, GROUP>(a, a.items[a.first[ST] + (int)blockIdx.x], threadIdx.x, smem);
 }
 
 // The whole step in one cooperative launch (all blocks resident): block b
@@ -324,9 +317,8 @@ int build_items(evx_batch_plan* p) {
       int64_t nt = 0;
       switch (s) {
         case 0: {
-          constexpr int BY = NTY * TileCfg<T>::PY;
-          b.tg.ntz = (int)cdiv(b.nz, BZ);
-          b.tg.nty = (int)cdiv(b.ny, BY);
+          b.tg.ntz = (int)cdiv(b.nz, ChB::TZ);
+          b.tg.nty = (int)cdiv(b.ny, ChB::BY);
           b.tg.xc = p->xchunk < b.nx ? p->xchunk : b.nx;
           b.tg.nxc = (int)cdiv(b.nx, b.tg.xc);
           nt = (int64_t)b.tg.ntz * b.tg.nty * b.tg.nxc;
@@ -422,15 +414,21 @@ int launch_coop(const BArgs& a, hipStream_t s) {
 int launch_step(evx_batch_plan* p, void* state, void* ws, hipStream_t s) {
   const BArgs a = make_args(p, state, ws);
   if (p->one_launch) return p->fft_group > 1 ? launch_coop<true>(a, s) : launch_coop<false>(a, s);
-  for (int st = 0; st < NSTAGE; ++st) {
+  const bool group = p->fft_group > 1;
+  using K = void (*)(BArgs);
+  auto launch = [&](int st, K one, K grouped) -> int {
     const int n = p->stage_first[st + 1] - p->stage_first[st];
-    if (n == 0) continue;
-    if (st > 0 && p->fft_group > 1)
-      hipLaunchKernelGGL(batch_stage<true>, dim3(n), dim3(BT), 0, s, a, p->stage_first[st]);
-    else
-      hipLaunchKernelGGL(batch_stage<false>, dim3(n), dim3(BT), 0, s, a, p->stage_first[st]);
-    EVX_TRY(check_launch("batch_stage"));
-  }
+    if (n == 0) return EVX_OK;
+    const K kernel = group ? grouped : one;
+    hipLaunchKernelGGL(kernel, dim3(n), dim3(BT), 0, s, a);
+    return check_launch("batch_stage");
+  };
+  EVX_TRY(launch(0, batch_stage<0, false>, batch_stage<0, false>));
+  EVX_TRY(launch(1, batch_stage<1, false>, batch_stage<1, true>));
+  EVX_TRY(launch(2, batch_stage<2, false>, batch_stage<2, true>));
+  EVX_TRY(launch(3, batch_stage<3, false>, batch_stage<3, true>));
+  EVX_TRY(launch(4, batch_stage<4, false>, batch_stage<4, true>));
+  EVX_TRY(launch(5, batch_stage<5, false>, batch_stage<5, true>));
   return EVX_OK;
 }
 

@@ -69,6 +69,12 @@ struct ChCoef {
     return D * dv;                                                                                        \
   }
 
+// Fused multiply-add written out.  The contracted formulas name every one of
+// them, so that each kernel instance that evaluates them (short and long
+// chunks, fused and separate sweeps) rounds alike.
+__device__ __forceinline__ float fused(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double fused(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
 template <bool STRICT>
 struct Ops;
 template <>
@@ -101,8 +107,9 @@ struct Ops<false> {
   }
   template <typename T>
   static __device__ __forceinline__ T flux_q(T q_lo, T c_hi, T m_lo, T m_hi) {
+#pragma clang fp contract(off)
     const T t = q_lo - c_hi;
-    return (T(1) - t * t) * (m_hi - m_lo);
+    return fused(-t, t, T(1)) * (m_hi - m_lo);
   }
   template <typename T>
   static __device__ __forceinline__ T flux(T c_lo, T c_hi, T m_lo, T m_hi, T /*id*/) {
@@ -146,13 +153,15 @@ __host__ __device__ inline ChW<T> ch_weights(const Geo<T>& g, const ChCoef<T>& k
 // Ops<false>::mu and Ops<false>::div with folded weights.
 template <typename T>
 __device__ __forceinline__ T mu_w(T c, T xp, T xm, T yp, T ym, T zp, T zm, const ChW<T>& W) {
-  const T l = (((xp + xm) * W.wx + (yp + ym) * W.wy) + (zp + zm) * W.wz) - c * W.wc;
-  const T p = (T(2) * c - T(3)) * c + T(1);
-  return (W.s18 * c) * p - l;
+#pragma clang fp contract(off)
+  const T l = fused(-c, W.wc, fused(zp + zm, W.wz, fused(yp + ym, W.wy, (xp + xm) * W.wx)));
+  const T p = fused(fused(T(2), c, T(-3)), c, T(1));
+  return fused(W.s18 * c, p, -l);
 }
 template <typename T>
 __device__ __forceinline__ T div_w(T fxm, T fxp, T fym, T fyp, T fzm, T fzp, const ChW<T>& W) {
-  return ((fxp - fxm) * W.dx + (fyp - fym) * W.dy) + (fzp - fzm) * W.dz;
+#pragma clang fp contract(off)
+  return fused(fzp - fzm, W.dz, fused(fyp - fym, W.dy, (fxp - fxm) * W.dx));
 }
 
 // Strict-order shorthands used by code that must match the reference rounding.

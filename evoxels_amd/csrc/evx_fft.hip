@@ -228,11 +228,6 @@ namespace {
 // upload): the first step on a new grid shape pays for them.
 template <typename T>
 int make_twiddles(AxisHost (&ax)[3], void** buf) {
-  const long double tau = 6.283185307179586476925286766559005768L;
-  auto root = [&](int64_t j, int64_t n) {
-    const long double ang = tau * (long double)(j % n) / (long double)n;
-    return cpx<T>{static_cast<T>(cosl(ang)), static_cast<T>(-sinl(ang))};
-  };
   auto aligned = [](size_t n) { return (n + 15) & ~size_t(15); };
   size_t total = 0;
   for (const AxisHost& h : ax) total += aligned(h.n) + aligned(h.line.tab);
@@ -242,13 +237,25 @@ int make_twiddles(AxisHost (&ax)[3], void** buf) {
     return fail(EVX_ERR_NOMEM, "hipMalloc of %zu twiddles failed", total);
   }
   size_t at = 0;
-  for (AxisHost& h : ax) {
-    for (int m = 0; m < h.n; ++m) t[at + m] = root(m, h.n);
+  const long double tau = 6.283185307179586476925286766559005768L;
+  for (int a = 0; a < 3; ++a) {
+    AxisHost& h = ax[a];
     h.tw = static_cast<cpx<T>*>(*buf) + at;
-    at += aligned(h.n);
-    line_fill_table(h.line, t.data() + at, root);
-    h.ltab = static_cast<cpx<T>*>(*buf) + at;
-    at += aligned(h.line.tab);
+    h.ltab = static_cast<cpx<T>*>(*buf) + at + aligned(h.n);
+    cpx<T>* const root = t.data() + at;
+    int same = 0;  // an earlier axis of the same length
+    while (same < a && ax[same].n != h.n) ++same;
+    if (same < a) {
+      std::copy_n(t.data() + (static_cast<cpx<T>*>(ax[same].tw) - static_cast<cpx<T>*>(*buf)),
+                  aligned(h.n) + aligned(h.line.tab), root);
+    } else {
+      for (int m = 0; m < h.n; ++m) {
+        const long double ang = tau * (long double)m / (long double)h.n;
+        root[m] = cpx<T>{static_cast<T>(cosl(ang)), static_cast<T>(-sinl(ang))};
+      }
+      line_fill_table(h.line, root + aligned(h.n), [&](int64_t j, int64_t q) { return root[j % q * (h.n / q)]; });
+    }
+    at += aligned(h.n) + aligned(h.line.tab);
   }
   if (hipMemcpy(*buf, t.data(), sizeof(cpx<T>) * total, hipMemcpyHostToDevice) != hipSuccess)
     return fail(EVX_ERR_HIP, "twiddle upload failed");

@@ -140,13 +140,20 @@ __global__ __launch_bounds__(NT) void gs_rhs_kernel(const T* __restrict__ u, T* 
   }
 }
 
-template <typename T, bool STRICT>
+template <typename T>
 __global__ __launch_bounds__(NT) void ch_rhs_kernel(const T* __restrict__ u, T* __restrict__ out, Dims d, Bc bc,
-                                                    Geo<T> g, ChCoef<T> k, Epi ep, TileGrid tg,
-                                                    const double* __restrict__ chan, unsigned tile_base) {
+                                                    Geo<T> g, ChCoef<T> k, Epi ep, TileGrid tg) {
   __shared__ __align__(16) unsigned char smem[ChTile<T>::LDS_BYTES];
-  ch_rhs_tile<T, STRICT>(u, out, d, bc, g, k, ep, tg, chan, tile_base + xcd_tile(blockIdx.x, gridDim.x),
-                         threadIdx.y * BZ + threadIdx.x, smem);
+  ch_rhs_tile<T>(u, out, d, bc, g, k, ep, tg, xcd_tile(blockIdx.x, gridDim.x), threadIdx.y * BZ + threadIdx.x, smem);
+}
+
+template <typename T, int TZ, int PY, bool SHORT>
+__global__ __launch_bounds__(NT) void ch_periodic_kernel(const T* __restrict__ u, T* __restrict__ out, Dims d,
+                                                         Geo<T> g, ChCoef<T> k, TileGrid tg,
+                                                         const double* __restrict__ chan, unsigned tile_base) {
+  __shared__ __align__(16) unsigned char smem[ChPer<T, TZ, PY>::LDS_BYTES];
+  ch_periodic_tile<T, TZ, PY, SHORT>(u, out, d, g, k, tg, chan, tile_base + xcd_tile(blockIdx.x, gridDim.x), threadIdx.x,
+                                 smem);
 }
 
 // ---------------------------------------------------------------------------
@@ -523,27 +530,48 @@ int launch_gs(const void* u, void* out, const Dims& d, const Bc& bc, const evx_g
   return check_launch("gs_rhs_kernel");
 }
 
+template <typename T>
+int launch_ch(const void* u, void* out, const Dims& d, const Bc& bc, const evx_grid* g, double eps,
+              double D, const Epi& ep, hipStream_t s) {
+  TileGrid tg;
+  dim3 grid = stencil_grid<T>(d, &tg, EVX_RESIDENT_ROUND(ch_rhs_kernel<T>));
+  ChCoef<T> k{static_cast<T>(18.0 / eps), static_cast<T>(2.0 * eps), static_cast<T>(D)};
+  hipLaunchKernelGGL(ch_rhs_kernel<T>, grid, dim3(BZ, NTY), 0, s, static_cast<const T*>(u), static_cast<T*>(out), d,
+                     bc, make_geo<T>(g), k, ep, tg);
+  return check_launch("ch_rhs_kernel");
+}
+
 constexpr int SLAB_XCHUNK = 16;
 
-template <typename T, bool STRICT = true>
-int launch_ch(const void* u, void* out, const Dims& d, const Bc& bc, const evx_grid* g, double eps,
-              double D, const Epi& ep, hipStream_t s, const double* chan = nullptr, int64_t xa = 0,
-              int64_t xb = -1) {
+// Tile of the periodic float32 right-hand side: 16 x 64 points on large grids
+// whose z length wastes no more of a 64-wide tile than of a 32-wide one, else
+// 16 x 32 (MI355X, us, 64 / 32 wide: 512^3 265 / 305, 16 x 128^3 81 / 86,
+// 256^3 36.4 / 36.4, 200^3 30.2 / 27.1, 300x270x350 64.7 / 63.7, 32^3 9.0 / 7.0).
+// Float64 tiles are 16 x 32 (400^3 285 / 257, 4 x 96^3 26 / 22).
+inline bool ch_wide_tile(const Dims& d) {
+  return (d.nz + 63) / 64 * 2 == (d.nz + 31) / 32 && d.c * d.vol() >= (int64_t(1) << 24);
+}
+
+template <typename T, int TZ, int PY>
+int launch_ch_periodic(const T* u, T* out, const Dims& d, const Geo<T>& g, const ChCoef<T>& k, const double* chan,
+                       int64_t xa, int64_t xb, hipStream_t s) {
+  constexpr int BY = ChPer<T, TZ, PY>::BY;
   TileGrid tg;
-  dim3 grid = stencil_grid<T>(d, &tg, EVX_RESIDENT_ROUND((ch_rhs_kernel<T, STRICT>)));
-  unsigned base = 0;
+  tg.ntz = (int)((d.nz + TZ - 1) / TZ);
+  tg.nty = (int)((d.ny + BY - 1) / BY);
+  const int64_t per_chunk = (int64_t)tg.ntz * tg.nty;
+  tg.xc = xb >= 0 ? SLAB_XCHUNK
+                  : balanced_xchunk(d.nx, per_chunk * d.c, EVX_RESIDENT_ROUND((ch_periodic_kernel<T, TZ, PY, false>)), 4);
+  tg.nxc = (int)((d.nx + tg.xc - 1) / tg.xc);
+  unsigned base = 0, blocks = (unsigned)(per_chunk * tg.nxc * d.c);
   if (xb >= 0) {  // x-slab [xa, xb) of a one-channel field, at tile-chunk granularity
-    tg.xc = SLAB_XCHUNK;
-    tg.nxc = (int)((d.nx + tg.xc - 1) / tg.xc);
-    const int64_t per_chunk = (int64_t)tg.ntz * tg.nty;
     const int64_t ca = xa / tg.xc, cb = (xb + tg.xc - 1) / tg.xc;
     base = (unsigned)(ca * per_chunk);
-    grid = dim3((unsigned)((cb - ca) * per_chunk));
+    blocks = (unsigned)((cb - ca) * per_chunk);
   }
-  ChCoef<T> k{static_cast<T>(18.0 / eps), static_cast<T>(2.0 * eps), static_cast<T>(D)};
-  hipLaunchKernelGGL((ch_rhs_kernel<T, STRICT>), grid, dim3(BZ, NTY), 0, s, static_cast<const T*>(u),
-                     static_cast<T*>(out), d, bc, make_geo<T>(g), k, ep, tg, chan, base);
-  return check_launch("ch_rhs_kernel");
+  auto kernel = tg.xc <= CH_SHORT ? ch_periodic_kernel<T, TZ, PY, true> : ch_periodic_kernel<T, TZ, PY, false>;
+  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(NT), 0, s, u, out, d, g, k, tg, chan, base);
+  return check_launch("ch_periodic_kernel");
 }
 
 template <typename T>
@@ -579,8 +607,15 @@ int stencil_rhs_ch_periodic(int32_t dtype, const void* u, void* out, const Dims&
   const Epi ep{EVX_OUT_RHS, 0.0, nullptr, nullptr, nullptr};
   if (d.ny * d.nz * (dtype == EVX_F32 ? 4 : 8) >= (int64_t(1) << 32))
     return fail(EVX_ERR_UNSUPPORTED, "a (y,z) plane of more than 4 GiB");
-  return dtype == EVX_F32 ? launch_ch<float, false>(u, out, d, b, &g, eps, D, ep, s, chan, xa, xb)
-                          : launch_ch<double, false>(u, out, d, b, &g, eps, D, ep, s, chan, xa, xb);
+  if (dtype == EVX_F32) {
+    const Geo<float> q = make_geo<float>(&g);
+    const ChCoef<float> k{static_cast<float>(18.0 / eps), static_cast<float>(2.0 * eps), static_cast<float>(D)};
+    auto launch = ch_wide_tile(d) ? launch_ch_periodic<float, 64, 4> : launch_ch_periodic<float, 32, 2>;
+    return launch(static_cast<const float*>(u), static_cast<float*>(out), d, q, k, chan, xa, xb, s);
+  }
+  const ChCoef<double> k{18.0 / eps, 2.0 * eps, D};
+  return launch_ch_periodic<double, 32, 2>(static_cast<const double*>(u), static_cast<double*>(out), d,
+                                           make_geo<double>(&g), k, chan, xa, xb, s);
 }
 
 // x-planes per CH tile chunk of slab launches (slabs start on a multiple of

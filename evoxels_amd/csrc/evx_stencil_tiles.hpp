@@ -262,10 +262,10 @@ struct TileOrigin {
   int64_t z0, y0, x0, x1, ch;
 };
 
-template <int BY>
+template <int BY, int TZ = BZ>
 __host__ __device__ __forceinline__ TileOrigin tile_origin(const TileGrid& tg, const Dims& d, unsigned t) {
   TileOrigin o;
-  o.z0 = (int64_t)(t % tg.ntz) * BZ;
+  o.z0 = (int64_t)(t % tg.ntz) * TZ;
   t /= tg.ntz;
   o.y0 = (int64_t)(t % tg.nty) * BY;
   t /= tg.nty;
@@ -290,18 +290,44 @@ __host__ inline int pick_xchunk(const Dims& d, int64_t tiles_yz, int64_t target 
   return (int)xc;
 }
 
+// Planes per chunk of a streaming launch of tiles_yz tiles (all channels), on a
+// device that holds `resident` blocks at once: the chunk that minimises
+// rounds * (planes + warm), `warm` the warm-up of a chunk in planes.  A launch
+// just above a whole number of rounds pays a whole round for its tail: the
+// 300x270x350 float32 right-hand side took 81 us with 1326 blocks on 1280
+// slots, 65 us with 19 planes more evenly split (MI355X).
+__host__ inline int balanced_xchunk(int64_t nx, int64_t tiles_yz, int64_t resident, int warm) {
+  int best = (int)nx;
+  double best_cost = 1e300;
+  for (int64_t nxc = 1; nxc <= nx; ++nxc) {
+    const int64_t xc = (nx + nxc - 1) / nxc;
+    if (nxc > 1 && (nx + nxc - 2) / (nxc - 1) == xc) continue;  // the same chunk length
+    const int64_t rounds = (tiles_yz * nxc + resident - 1) / resident;
+    const double cost = (double)rounds * (double)(xc + warm);
+    if (cost < best_cost) {
+      best_cost = cost;
+      best = (int)xc;
+    }
+    if (nxc > 64 && tiles_yz * nxc > 8 * resident) break;
+  }
+  return best;
+}
+
 // Tile grid of a streaming stencil launch of about `target` blocks; returns
 // the block count (tiles over z, y, x-chunks and channels).
-template <typename T>
-__host__ inline unsigned stencil_tiles(const Dims& d, TileGrid* tg, int64_t target) {
-  constexpr int BY = NTY * TileCfg<T>::PY;
-  const int64_t ty = (d.ny + BY - 1) / BY, tzn = (d.nz + BZ - 1) / BZ;
+template <int BY, int TZ>
+__host__ inline unsigned stencil_tiles_of(const Dims& d, TileGrid* tg, int64_t target) {
+  const int64_t ty = (d.ny + BY - 1) / BY, tzn = (d.nz + TZ - 1) / TZ;
   tg->xc = pick_xchunk(d, ty * tzn, target);
   const int64_t nxc = (d.nx + tg->xc - 1) / tg->xc;
   tg->ntz = (int)tzn;
   tg->nty = (int)ty;
   tg->nxc = (int)nxc;
   return (unsigned)(tzn * ty * nxc * d.c);
+}
+template <typename T>
+__host__ inline unsigned stencil_tiles(const Dims& d, TileGrid* tg, int64_t target) {
+  return stencil_tiles_of<NTY * TileCfg<T>::PY, BZ>(d, tg, target);
 }
 
 // ---------------------------------------------------------------------------
@@ -331,17 +357,13 @@ struct ChTile {
 
 // One (y,z) tile x x-chunk of the CH right-hand side.  tid = flat thread index
 // in a 256-thread block, tile = flat tile index (see tile_origin), smem =
-// ChTile<T>::LDS_BYTES of LDS.  The contracted flavour (!STRICT) serves the
-// fully periodic semi-implicit path only: it has no ghost logic, loads
-// through PeriodicLoader and stores the plain right-hand side with 32-bit
-// in-plane offsets whatever ep says (its callers pass EVX_OUT_RHS).
-template <typename T, bool STRICT>
+// ChTile<T>::LDS_BYTES of LDS.
+template <typename T>
 __device__ __forceinline__ void ch_rhs_tile(const T* __restrict__ u, T* __restrict__ out, const Dims& d,
                                             const Bc& bc, const Geo<T>& g, ChCoef<T> k, const Epi& ep,
-                                            const TileGrid& tg, const double* __restrict__ chan, unsigned tile,
-                                            int tid, unsigned char* smem) {
+                                            const TileGrid& tg, unsigned tile, int tid, unsigned char* smem) {
 #pragma clang fp contract(off)
-  using Op = Ops<STRICT>;
+  using Op = Ops<true>;
   using TC = ChTile<T>;
   constexpr int PY = TC::PY, BY = TC::BY;
   constexpr int CW = TC::CW, CR = TC::CR, NC = TC::NC;
@@ -354,13 +376,8 @@ __device__ __forceinline__ void ch_rhs_tile(const T* __restrict__ u, T* __restri
   const int64_t z0 = o.z0, y0 = o.y0, x0 = o.x0, x1 = o.x1;
   const T* uc = u + o.ch * d.vol();
   T* oc = out + o.ch * d.vol();
-  if (chan) {  // per-channel (eps, D), rounded as the host rounds the scalars
-    const double e = chan[2 * o.ch], dd = chan[2 * o.ch + 1];
-    k = ChCoef<T>{static_cast<T>(18.0 / e), static_cast<T>(2.0 * e), static_cast<T>(dd)};
-  }
-  constexpr bool PER = !STRICT;
-  const bool xper = PER || bc.kind[0] == EVX_BC_PERIODIC;
-  const bool yper = PER || bc.kind[1] == EVX_BC_PERIODIC, zper = PER || bc.kind[2] == EVX_BC_PERIODIC;
+  const bool xper = bc.kind[0] == EVX_BC_PERIODIC;
+  const bool yper = bc.kind[1] == EVX_BC_PERIODIC, zper = bc.kind[2] == EVX_BC_PERIODIC;
   const int r0 = ty * PY;
   const int64_t gz = z0 + tz;
 
@@ -461,22 +478,10 @@ __device__ __forceinline__ void ch_rhs_tile(const T* __restrict__ u, T* __restri
     }
   };
 
-  using Loader = typename std::conditional<PER, PeriodicLoader<T, 2, CR, CW, true>,
-                                           PlaneLoader<T, 2, CR, CW, true>>::type;
-  Loader pl;
-  auto pl_init = [&]() {
-    if constexpr (PER) pl.init(y0, z0, d, tid);
-    else pl.init(y0, z0, d, bc, tid);
-  };
-  auto pl_fetch = [&](int64_t xg) {
-    if constexpr (PER) pl.fetch(uc, xg, d);
-    else pl.fetch(uc, xg, d, bc);
-  };
-  auto pl_commit = [&](int slot) {
-    if constexpr (PER) pl.commit(&cs[slot][0][0], tid);
-    else pl.commit(&cs[slot][0][0], bc, tid);
-  };
-  pl_init();
+  PlaneLoader<T, 2, CR, CW, true> pl;
+  auto pl_fetch = [&](int64_t xg) { pl.fetch(uc, xg, d, bc); };
+  auto pl_commit = [&](int slot) { pl.commit(&cs[slot][0][0], bc, tid); };
+  pl.init(y0, z0, d, bc, tid);
   const int b = tz + 2, bm = tz + 1;
   // Warm-up: planes x0-2 .. x0+1, mu(x0-1) and mu(x0), and the flux through
   // the x face x0-1/2 (afterwards carried in registers, so neither c(x-1)
@@ -505,11 +510,6 @@ __device__ __forceinline__ void ch_rhs_tile(const T* __restrict__ u, T* __restri
   if (x0 + 3 <= x1 + 1) pl_fetch(x0 + 3);
   __syncthreads();  // mu(x0+1) below reuses the slot of mu(x0-1) read above
   const int64_t plane = d.ny * d.nz;
-  // plain right-hand-side stores of the periodic flavour: 32-bit byte offset
-  // of this thread's first row in the plane, rows nz apart
-  const bool full_tile = y0 + BY <= d.ny && z0 + BZ <= d.nz;
-  const uint32_t obyte0 = static_cast<uint32_t>(((y0 + r0) * d.nz + gz) * (int64_t)sizeof(T));
-  const uint32_t orow_bytes = static_cast<uint32_t>(d.nz * (int64_t)sizeof(T));
   for (int64_t x = x0; x < x1; ++x) {
     // mu(x+1) from c(x), c(x+1), c(x+2), into the slot of mu(x-1)
     compute_mu(x + 1);
@@ -518,51 +518,229 @@ __device__ __forceinline__ void ch_rhs_tile(const T* __restrict__ u, T* __restri
     const T(*Cp)[CW] = cs[ring<NC>(x + 1 - x0 + 2)];
     const T(*M0)[MW] = ms[ring<NM>(x - x0 + 1)];
     const T(*Mp)[MW] = ms[ring<NM>(x + 1 - x0 + 1)];
-    T cc[PY + 2], mc[PY + 2], fy[PY + 1], qc[PY + 1];
+    T cc[PY + 2], mc[PY + 2], fy[PY + 1];
 #pragma unroll
     for (int j = 0; j < PY + 2; ++j) {
       cc[j] = C0[r0 + j + 1][b];
       mc[j] = M0[r0 + j][bm];
     }
-    if constexpr (PER) {  // q = 1 - c of each own point, shared by its faces
 #pragma unroll
-      for (int j = 0; j <= PY; ++j) qc[j] = T(1) - cc[j];
-    }
-#pragma unroll
-    for (int j = 0; j <= PY; ++j) {
-      if constexpr (PER) fy[j] = Op::flux_q(qc[j], cc[j + 1], mc[j], mc[j + 1]);
-      else fy[j] = Op::flux(cc[j], cc[j + 1], mc[j], mc[j + 1], g.idy);
-    }
+    for (int j = 0; j <= PY; ++j) fy[j] = Op::flux(cc[j], cc[j + 1], mc[j], mc[j + 1], g.idy);
 #pragma unroll
     for (int q = 0; q < PY; ++q) {
       const int a = r0 + q + 2, am = r0 + q + 1;
       const T c0 = cc[q + 1], m0 = mc[q + 1];
-      T fxp, fzm, fzp;
-      if constexpr (PER) {
-        const T q0 = qc[q + 1];
-        fxp = Op::flux_q(q0, Cp[a][b], m0, Mp[am][bm]);
-        fzm = Op::flux_q(q0, C0[a][b - 1], M0[am][bm - 1], m0);
-        fzp = Op::flux_q(q0, C0[a][b + 1], m0, M0[am][bm + 1]);
-      } else {
-        fxp = Op::flux(c0, Cp[a][b], m0, Mp[am][bm], g.idx);
-        fzm = Op::flux(C0[a][b - 1], c0, M0[am][bm - 1], m0, g.idz);
-        fzp = Op::flux(c0, C0[a][b + 1], m0, M0[am][bm + 1], g.idz);
-      }
+      const T fxp = Op::flux(c0, Cp[a][b], m0, Mp[am][bm], g.idx);
+      const T fzm = Op::flux(C0[a][b - 1], c0, M0[am][bm - 1], m0, g.idz);
+      const T fzp = Op::flux(c0, C0[a][b + 1], m0, M0[am][bm + 1], g.idz);
       const T r = Op::div(carry[q], fxp, fy[q], fy[q + 1], fzm, fzp, g, k.D);
       carry[q] = fxp;
       const int64_t gy = y0 + r0 + q;
-      if constexpr (PER) {  // the contracted flavour's callers all take the plain right-hand side
-        if (full_tile || (gy < d.ny && gz < d.nz))
-          *reinterpret_cast<T*>(reinterpret_cast<char*>(oc + x * plane) + (obyte0 + q * orow_bytes)) = r;
-      } else if (gy < d.ny && gz < d.nz) {
-        epilogue(ep, uc, oc, x * plane + gy * d.nz + gz, r);
-      }
+      if (gy < d.ny && gz < d.nz) epilogue(ep, uc, oc, x * plane + gy * d.nz + gz, r);
     }
     // plane x+3 (fetched one iteration ago) goes to the slot of c(x-1), which
     // neither the output above nor mu(x+1) reads; it feeds mu(x+2)
     if (x + 3 <= x1 + 1) pl_commit(ring<NC>(x + 3 - x0 + 2));
     if (x + 4 <= x1 + 1) pl_fetch(x + 4);
     __syncthreads();
+  }
+}
+
+// ---------------------------------------------------------------------------
+// The same right-hand side on a fully periodic grid, written plainly (the
+// semi-implicit path): no ghost logic, contracted algebra.  A block owns a
+// (BY x TZ) tile of (y, z) and an x-chunk; thread (ty, tz) owns PY rows of one
+// column and keeps c(x), c(x+1), c(x+2), mu(x), mu(x+1) and the flux through
+// the face x-1/2 of its points in registers, so only y and z neighbours come
+// from LDS (a ring of four c planes and two mu planes) and a plane takes one
+// barrier: plane x+3 is written to the fourth slot and mu(x+1) to the second
+// while c(x), c(x+1), c(x+2) and mu(x) are read.
+//
+// The planes of the warm-up are fetched together (one memory latency instead
+// of one per plane); SHORT, for chunks of at most CH_SHORT planes, fetches
+// every plane of the chunk that way.
+//
+// Bound by vector issue on large grids (64 vector instructions per point and
+// plane with 16 x 32 tiles, 57 with 16 x 64) and by the chain of planes on
+// small ones.  MI355X, us, before (two barriers a plane, neighbours of both
+// fields from LDS) -> now: 32^3 float32 12.4 -> 5.2, 100^3 float64 13.8 -> 11,
+// 4 x 96^3 float64 36 -> 21, 300x270x350 float32 92 -> 62, 400^3 float64
+// 394 -> 267, 512^3 float32 282 -> 262.
+// ---------------------------------------------------------------------------
+constexpr int CH_SHORT = 4;
+
+template <typename T, int TZ_, int PY_>
+struct ChPer {
+  static constexpr int TZ = TZ_, NR = NT / TZ;  // tile width, thread rows
+  static constexpr int PY = PY_, BY = NR * PY;
+  static constexpr int CW = TZ + 4, CR = BY + 4, NC = 4;
+  static constexpr int MW = TZ + 2, MR = BY + 2, NM = 2;
+  static constexpr int NHALO = 2 * TZ + 2 * BY;  // mu points on rows -1, BY and columns -1, TZ
+  static constexpr size_t LDS_BYTES = sizeof(T) * (NC * CR * CW + NM * MR * MW);
+  static_assert(NHALO <= NT, "one mu halo point per thread");
+};
+
+template <typename T, int TZ, int PYT, bool SHORT>
+__device__ __forceinline__ void ch_periodic_tile(const T* __restrict__ u, T* __restrict__ out, const Dims& d,
+                                                 const Geo<T>& g, ChCoef<T> k, const TileGrid& tg,
+                                                 const double* __restrict__ chan, unsigned tile, int tid,
+                                                 unsigned char* smem) {
+  using P = ChPer<T, TZ, PYT>;
+  using Op = Ops<false>;
+  constexpr int PY = P::PY, BY = P::BY, CW = P::CW, MW = P::MW;
+  constexpr int CS = P::CR * CW, MS = P::MR * MW;
+  using Loader = PeriodicLoader<T, 2, P::CR, CW, true>;
+  constexpr int NPT = Loader::NPT;
+  T* const cs = reinterpret_cast<T*>(smem);
+  T* const ms = cs + P::NC * CS;
+  const int tz = tid % TZ, r0 = tid / TZ * PY;
+  const TileOrigin o = tile_origin<BY, TZ>(tg, d, tile);
+  const int64_t x0 = o.x0;
+  const int nxp = (int)(o.x1 - x0);  // planes of the chunk
+  const T* const uc = u + o.ch * d.vol();
+  if (chan) {  // per-channel (eps, D), rounded as the host rounds the scalars
+    const double e = chan[2 * o.ch], dd = chan[2 * o.ch + 1];
+    k = ChCoef<T>{static_cast<T>(18.0 / e), static_cast<T>(2.0 * e), static_cast<T>(dd)};
+  }
+  const ChW<T> W = ch_weights(g, k);
+  const int oc = (r0 + 2) * CW + tz + 2, om = (r0 + 1) * MW + tz + 1;
+  // this thread's mu halo point: offset of its c point in a c plane and of itself in a mu plane
+  int hc = 0, hm = 0;
+  const bool halo = tid < P::NHALO;
+  if (halo) {
+    int y, z;
+    if (tid < 2 * TZ) {
+      y = tid < TZ ? -1 : BY;
+      z = tid % TZ;
+    } else {
+      const int h = tid - 2 * TZ;
+      y = h % BY;
+      z = h < BY ? -1 : TZ;
+    }
+    hc = (y + 2) * CW + z + 2;
+    hm = (y + 1) * MW + z + 1;
+  }
+  Loader pl;
+  pl.init(o.y0, o.z0, d, tid);
+  // fetch() loads the planes x0-2, x0-1, ... in turn: the wrapped index is
+  // advanced by a compare (a modulo per plane is a 64-bit division)
+  const int nx = (int)d.nx;
+  int xw = (int)x0 - 2;
+  while (xw < 0) xw += nx;
+  auto fetch = [&](T(&v)[NPT]) {
+    const char* p = reinterpret_cast<const char*>(uc + (int64_t)xw * (d.ny * d.nz));
+#pragma unroll
+    for (int q = 0; q < NPT; ++q)
+      if (pl.valid(q)) v[q] = *reinterpret_cast<const T*>(p + pl.boff[q]);
+    xw = xw + 1 == nx ? 0 : xw + 1;
+  };
+  auto commit = [&](int slot, const T(&v)[NPT]) {
+    T* const c = cs + slot * CS;
+#pragma unroll
+    for (int q = 0; q < NPT; ++q)
+      if (pl.valid(q)) c[tid + q * NT] = clip01(v[q]);
+  };
+  // mu of the own points of plane slot C with x neighbours xm, xp
+  auto mu_own = [&](const T* C, const T(&c)[PY], const T(&xm)[PY], const T(&xp)[PY], T(&m)[PY]) {
+    const T lo = C[oc - CW], hi = C[oc + PY * CW];
+#pragma unroll
+    for (int q = 0; q < PY; ++q)
+      m[q] = mu_w(c[q], xp[q], xm[q], q + 1 < PY ? c[q + 1 < PY ? q + 1 : q] : hi, q > 0 ? c[q > 0 ? q - 1 : q] : lo,
+                  C[oc + q * CW + 1], C[oc + q * CW - 1], W);
+  };
+  auto mu_halo = [&](const T* Cm, const T* C, const T* Cp, T* M) {
+    if (halo)
+      M[hm] = mu_w(C[hc], Cp[hc], Cm[hc], C[hc + CW], C[hc - CW], C[hc + 1], C[hc - 1], W);
+  };
+
+  // warm-up: planes x0-2 .. x0+3 (SHORT: to the chunk's last) in flight together
+  constexpr int PRE = SHORT ? CH_SHORT + 4 : 6;
+  T w[PRE][NPT];
+#pragma unroll
+  for (int p = 0; p < PRE; ++p)
+    if (p < 5 || p <= nxp + 3) fetch(w[p]);
+#pragma unroll
+  for (int p = 0; p < 4; ++p) commit(p, w[p]);
+  __syncthreads();
+  T c0[PY], c1[PY], m0[PY], carry[PY];
+  {
+    T a[PY], b[PY], mp[PY];
+#pragma unroll
+    for (int q = 0; q < PY; ++q) {
+      a[q] = cs[oc + q * CW];
+      b[q] = cs[CS + oc + q * CW];
+      c0[q] = cs[2 * CS + oc + q * CW];
+      c1[q] = cs[3 * CS + oc + q * CW];
+    }
+    mu_own(cs + CS, b, a, c0, mp);
+    mu_own(cs + 2 * CS, c0, b, c1, m0);
+#pragma unroll
+    for (int q = 0; q < PY; ++q) {
+      ms[om + q * MW] = m0[q];
+      carry[q] = Op::flux_q(T(1) - b[q], c0[q], mp[q], m0[q]);
+    }
+    mu_halo(cs + CS, cs + 2 * CS, cs + 3 * CS, ms);
+  }
+  __syncthreads();  // every read of plane x0-2 is done
+  commit(0, w[4]);
+  __syncthreads();
+
+  const int64_t plane = d.ny * d.nz;
+  const bool full = o.y0 + BY <= d.ny && o.z0 + TZ <= d.nz;
+  const int64_t gz = o.z0 + tz;
+  const uint32_t obyte = static_cast<uint32_t>(((o.y0 + r0) * d.nz + gz) * (int64_t)sizeof(T));
+  const uint32_t orow = static_cast<uint32_t>(d.nz * (int64_t)sizeof(T));
+  T* ox = out + o.ch * d.vol() + x0 * plane;
+  // output plane x0 + i; c(x0+i+3) is in v on entry (if the chunk needs it)
+  auto step = [&](int i, T(&v)[NPT]) {
+    const T* const C0 = cs + ((i + 2) & 3) * CS;
+    const T* const C1 = cs + ((i + 3) & 3) * CS;
+    const T* const C2 = cs + (i & 3) * CS;
+    const T* const M0 = ms + (i & 1) * MS;
+    T* const M1 = ms + ((i + 1) & 1) * MS;
+    if (i + 3 <= nxp + 1) commit((i + 1) & 3, v);
+    if (!SHORT && i + 4 <= nxp + 1) fetch(v);
+    T c2[PY], m1[PY];
+#pragma unroll
+    for (int q = 0; q < PY; ++q) c2[q] = C2[oc + q * CW];
+    mu_own(C1, c1, c0, c2, m1);
+#pragma unroll
+    for (int q = 0; q < PY; ++q) M1[om + q * MW] = m1[q];
+    mu_halo(C0, C1, C2, M1);
+    T fy[PY + 1];
+    {
+      const T cl = C0[oc - CW], ch = C0[oc + PY * CW], ml = M0[om - MW], mh = M0[om + PY * MW];
+      fy[0] = Op::flux_q(T(1) - cl, c0[0], ml, m0[0]);
+#pragma unroll
+      for (int q = 1; q < PY; ++q) fy[q] = Op::flux_q(T(1) - c0[q - 1], c0[q], m0[q - 1], m0[q]);
+      fy[PY] = Op::flux_q(T(1) - c0[PY - 1], ch, m0[PY - 1], mh);
+    }
+#pragma unroll
+    for (int q = 0; q < PY; ++q) {
+      const T q0 = T(1) - c0[q];
+      const T fxp = Op::flux_q(q0, c1[q], m0[q], m1[q]);
+      const T fzm = Op::flux_q(q0, C0[oc + q * CW - 1], M0[om + q * MW - 1], m0[q]);
+      const T fzp = Op::flux_q(q0, C0[oc + q * CW + 1], m0[q], M0[om + q * MW + 1]);
+      const T r = div_w(carry[q], fxp, fy[q], fy[q + 1], fzm, fzp, W);
+      carry[q] = fxp;
+      if (full || (o.y0 + r0 + q < d.ny && gz < d.nz))
+        *reinterpret_cast<T*>(reinterpret_cast<char*>(ox) + (obyte + q * orow)) = r;
+    }
+#pragma unroll
+    for (int q = 0; q < PY; ++q) {
+      c0[q] = c1[q];
+      c1[q] = c2[q];
+      m0[q] = m1[q];
+    }
+    ox += plane;
+    __syncthreads();
+  };
+  if constexpr (SHORT) {
+#pragma unroll
+    for (int i = 0; i < CH_SHORT; ++i)
+      if (i < nxp) step(i, w[i + 5 < PRE ? i + 5 : PRE - 1]);
+  } else {
+    for (int i = 0; i < nxp; ++i) step(i, w[5]);
   }
 }
 

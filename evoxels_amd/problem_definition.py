@@ -122,6 +122,10 @@ class ODE(ABC):
     # ---- fused-kernel protocol used by the time steppers -----------------
     fused = False
 
+    def fused_for(self, u) -> bool:
+        """Whether ``launch`` can evaluate a step's epilogue for the state ``u``."""
+        return self.fused
+
     def _own_rhs(self, cls) -> bool:
         """True while ``rhs`` is ``cls.rhs`` itself: neither replaced on the
         instance (the manufactured-solution driver assigns ``problem.rhs``,
@@ -482,10 +486,34 @@ class MultiPhaseAllenCahn(SemiLinearODE):
         return n_phases <= 8 and pot is MultiPhaseAllenCahn._calc_well_derivatives and \
             proj in (MultiPhaseAllenCahn._sloppy_simplex_projection, MultiPhaseAllenCahn._euclidean_simplex_projection)
 
+    def fused_for(self, u):
+        """Whether one kernel evaluates the right-hand side of ``u``: up to
+        eight phases, built-in projection and potential, scalar ghost rules."""
+        return isinstance(u, torch.Tensor) and u.dim() == 4 and self._kernel_path(u.shape[0]) and \
+            self._own_rhs(MultiPhaseAllenCahn) and self._one_launch(u)
+
+    def _one_launch(self, u):
+        values = [v for _, vals in self.bc if vals is not None for v in vals]
+        return self._kernel_bcs() and not any(isinstance(v, torch.Tensor) for v in values) and \
+            u.shape[2] * u.shape[3] < 2 ** 31
+
+    def launch(self, u, out, epilogue):
+        euclid = getattr(self.project_to_simplex, "__func__", None) is \
+            MultiPhaseAllenCahn._euclidean_simplex_projection
+        g = self._grid(u)
+        b = _lib.make_bc(self.bc, self.vg.convention)
+        _lib.call("evx_multiphase_ac_rhs", _lib.dtype_code(u.dtype), _lib.ptr(u), _lib.ptr(out), C.byref(g),
+                  C.byref(b), float(self.eps), float(self.gab), float(self.M), float(self.curvature), int(euclid),
+                  C.byref(epilogue), _lib.stream_handle(u.device))
+
     def rhs(self, t, phis):
         phis = self._check_state(phis)
         n = phis.shape[0]
-        if self._kernel_path(n):
+        if self._kernel_path(n) and self._one_launch(phis):
+            out = torch.empty_like(phis)
+            self.launch(phis, out, _lib.make_epilogue())
+            return out
+        if self._kernel_path(n):  # ghost values given as fields: pad between the kernels
             dt_code = _lib.dtype_code(phis.dtype)
             stream = _lib.stream_handle(phis.device)
             proj = torch.empty_like(phis)

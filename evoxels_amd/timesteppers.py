@@ -23,6 +23,12 @@ from .problem_definition import ODE, SemiLinearODE, CahnHilliard, ReactionDiffus
 State = Any
 
 
+def _fused_for(problem, u) -> bool:
+    """Whether the problem's kernel takes a step's epilogue for the state u."""
+    ask = getattr(problem, "fused_for", None)
+    return ask(u) if ask is not None else problem.fused
+
+
 class TimeStepper(ABC):
     """timesteppers.py:9-29."""
 
@@ -55,7 +61,7 @@ class ForwardEuler(TimeStepper):
         return self.problem.fused
 
     def step(self, t: float, u: State) -> State:
-        if self.problem.fused:
+        if _fused_for(self.problem, u):
             u = self.problem._check_state(u)
             out = torch.empty_like(u)
             self.problem.launch(u, out, _lib.make_epilogue(_lib.OUT_EULER, self.dt))
@@ -79,7 +85,7 @@ class RungeKutta4(TimeStepper):
         return self.problem.fused
 
     def step(self, t: float, u: State) -> State:
-        if not self.problem.fused:
+        if not _fused_for(self.problem, u):
             k1 = self.problem.rhs(t, u)
             k2 = self.problem.rhs(t + 0.5 * self.dt, u + 0.5 * self.dt * k1)
             k3 = self.problem.rhs(t + 0.5 * self.dt, u + 0.5 * self.dt * k2)

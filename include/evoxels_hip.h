@@ -170,6 +170,16 @@ int evx_multiphase_ac_rhs_padded(int32_t dtype, const void* phis, const void* pa
                                  void* out, const evx_grid* g, double eps, double gab,
                                  double M, double curvature, void* stream);
 
+/* The same right-hand side from the raw phases in one launch: projection
+ * (`euclidean` as in evx_simplex_project), ghost rules of `bc` on the projected
+ * phases, Laplacians and potential, with the step epilogue `e` (NULL: plain
+ * right-hand side) applied to the raw phases.  1 to 8 phases; `out` must not
+ * alias `phis`. */
+int evx_multiphase_ac_rhs(int32_t dtype, const void* phis, void* out, const evx_grid* g,
+                          const evx_bc* bc, double eps, double gab, double M,
+                          double curvature, int32_t euclidean, const evx_epilogue* e,
+                          void* stream);
+
 /* ReactionDiffusionSBM.rhs without the source term (problem_definition.py:
  * 273-287) from the padded field and the padded (clipped) mask:
  * r = D * sum_axes grad_face(grad_face(z) - to_face(z/m)*grad_face(m)) + norm*bc_flux,

@@ -9,6 +9,7 @@
 //
 // Floating-point contraction is off in this file so that every product and
 // sum rounds where the reference's eager torch expression rounds.
+#include "evx_explicit.hpp"
 #include "evx_stencil_tiles.hpp"
 
 #pragma clang fp contract(off)
@@ -16,129 +17,6 @@
 namespace evx {
 namespace {
 
-
-// ---------------------------------------------------------------------------
-// Reaction-diffusion (f == 0): r = D * laplace(pad_bc(u))
-// (problem_definition.py:226-229, fd_stencils.py:62-75)
-// ---------------------------------------------------------------------------
-template <typename T>
-__global__ __launch_bounds__(NT) void rd_rhs_kernel(const T* __restrict__ u, T* __restrict__ out, Dims d, Bc bc,
-                                                    Geo<T> g, T D, Epi ep, TileGrid tg) {
-  constexpr int PY = TileCfg<T>::PY, BY = NTY * PY;
-  constexpr int W = BZ + 2, ROWS = BY + 2, NR = 4;
-  __shared__ T cs[NR][ROWS][W];
-  const int tz = threadIdx.x, ty = threadIdx.y, tid = ty * BZ + tz;
-  const TileOrigin o = tile_origin<BY>(tg, d, xcd_tile(blockIdx.x, gridDim.x));
-  const int64_t z0 = o.z0, y0 = o.y0, x0 = o.x0, x1 = o.x1;
-  const T* uc = u + o.ch * d.vol();
-  T* oc = out + o.ch * d.vol();
-  PlaneLoader<T, 1, ROWS, W, false, true> pl;
-  pl.init(y0, z0, d, bc, tid);
-  for (int64_t xg = x0 - 1; xg <= x0 + 1; ++xg) {
-    pl.fetch(uc, xg, d, bc);
-    pl.commit(&cs[ring<NR>(xg - x0)][0][0], bc, tid);
-  }
-  if (x0 + 2 <= x1) pl.fetch(uc, x0 + 2, d, bc);
-  __syncthreads();
-  const int64_t plane = d.ny * d.nz;
-  const int64_t gz = z0 + tz;
-  for (int64_t x = x0; x < x1; ++x) {
-    // plane x+2 (fetched one iteration ago) goes to the slot of plane x-2
-    if (x + 2 <= x1) pl.commit(&cs[ring<NR>(x + 2 - x0)][0][0], bc, tid);
-    if (x + 3 <= x1) pl.fetch(uc, x + 3, d, bc);
-    const T(*Cm)[W] = cs[ring<NR>(x - 1 - x0)];
-    const T(*C0)[W] = cs[ring<NR>(x - x0)];
-    const T(*Cp)[W] = cs[ring<NR>(x + 1 - x0)];
-#pragma unroll
-    for (int q = 0; q < PY; ++q) {
-      const int yy = ty + NTY * q;
-      const int64_t gy = y0 + yy;
-      if (gy >= d.ny || gz >= d.nz) continue;
-      const int a = yy + 1, b = tz + 1;
-      const T c0 = C0[a][b];
-      const T lap = lap7(c0, Cp[a][b], Cm[a][b], C0[a + 1][b], C0[a - 1][b], C0[a][b + 1], C0[a][b - 1], g);
-      epilogue_v(ep, c0, oc, x * plane + gy * d.nz + gz, D * lap);
-    }
-    __syncthreads();
-  }
-}
-
-
-// ---------------------------------------------------------------------------
-// Two species with the Gray-Scott interaction a*b^2
-// (problem_definition.py:612-633):
-//   r_a = D_a*lap(a) - a*b^2 + F*(1 - a),   r_b = D_b*lap(b) + a*b^2 - k*b.
-// One block streams both species through their own plane rings, so the
-// interaction reads each value once; the tile grid has no channel dimension.
-// ---------------------------------------------------------------------------
-template <typename T>
-struct GsCoef {
-  T Da, Db, feed, kill;
-};
-
-template <typename T>
-__global__ __launch_bounds__(NT) void gs_rhs_kernel(const T* __restrict__ u, T* __restrict__ out, Dims d, Bc bc,
-                                                    Geo<T> g, GsCoef<T> k, Epi ep, TileGrid tg) {
-  constexpr int PY = TileCfg<T>::PY, BY = NTY * PY;
-  constexpr int W = BZ + 2, ROWS = BY + 2, NR = 4;
-  __shared__ T sa[NR][ROWS][W];
-  __shared__ T sb[NR][ROWS][W];
-  const int tz = threadIdx.x, ty = threadIdx.y, tid = ty * BZ + tz;
-  const TileOrigin o = tile_origin<BY>(tg, d, xcd_tile(blockIdx.x, gridDim.x));
-  const int64_t z0 = o.z0, y0 = o.y0, x0 = o.x0, x1 = o.x1;
-  const int64_t vol = d.vol();
-  const T* ua = u;
-  const T* ub = u + vol;
-  PlaneLoader<T, 1, ROWS, W, false, true> pa, pb;
-  pa.init(y0, z0, d, bc, tid);
-  pb.init(y0, z0, d, bc, tid);
-  for (int64_t xg = x0 - 1; xg <= x0 + 1; ++xg) {
-    pa.fetch(ua, xg, d, bc);
-    pb.fetch(ub, xg, d, bc);
-    pa.commit(&sa[ring<NR>(xg - x0)][0][0], bc, tid);
-    pb.commit(&sb[ring<NR>(xg - x0)][0][0], bc, tid);
-  }
-  if (x0 + 2 <= x1) {
-    pa.fetch(ua, x0 + 2, d, bc);
-    pb.fetch(ub, x0 + 2, d, bc);
-  }
-  __syncthreads();
-  const int64_t plane = d.ny * d.nz;
-  const int64_t gz = z0 + tz;
-  for (int64_t x = x0; x < x1; ++x) {
-    if (x + 2 <= x1) {
-      pa.commit(&sa[ring<NR>(x + 2 - x0)][0][0], bc, tid);
-      pb.commit(&sb[ring<NR>(x + 2 - x0)][0][0], bc, tid);
-    }
-    if (x + 3 <= x1) {
-      pa.fetch(ua, x + 3, d, bc);
-      pb.fetch(ub, x + 3, d, bc);
-    }
-    const T(*Am)[W] = sa[ring<NR>(x - 1 - x0)];
-    const T(*A0)[W] = sa[ring<NR>(x - x0)];
-    const T(*Ap)[W] = sa[ring<NR>(x + 1 - x0)];
-    const T(*Bm)[W] = sb[ring<NR>(x - 1 - x0)];
-    const T(*B0)[W] = sb[ring<NR>(x - x0)];
-    const T(*Bp)[W] = sb[ring<NR>(x + 1 - x0)];
-#pragma unroll
-    for (int q = 0; q < PY; ++q) {
-      const int yy = ty + NTY * q;
-      const int64_t gy = y0 + yy;
-      if (gy >= d.ny || gz >= d.nz) continue;
-      const int a = yy + 1, b = tz + 1;
-      const T av = A0[a][b], bv = B0[a][b];
-      const T la = lap7(av, Ap[a][b], Am[a][b], A0[a + 1][b], A0[a - 1][b], A0[a][b + 1], A0[a][b - 1], g);
-      const T lb = lap7(bv, Bp[a][b], Bm[a][b], B0[a + 1][b], B0[a - 1][b], B0[a][b + 1], B0[a][b - 1], g);
-      const T inter = av * (bv * bv);
-      const T ra = (k.Da * la - inter) + k.feed * (T(1) - av);
-      const T rb = (k.Db * lb + inter) - k.kill * bv;
-      const int64_t i = x * plane + gy * d.nz + gz;
-      epilogue_v(ep, av, out, i, ra);
-      epilogue_v(ep, bv, out, vol + i, rb);
-    }
-    __syncthreads();
-  }
-}
 
 template <typename T>
 __global__ __launch_bounds__(NT) void ch_rhs_kernel(const T* __restrict__ u, T* __restrict__ out, Dims d, Bc bc,
@@ -156,21 +34,6 @@ __global__ __launch_bounds__(NT) void ch_periodic_kernel(const T* __restrict__ u
                                  smem);
 }
 
-// ---------------------------------------------------------------------------
-// Two-phase Allen-Cahn (problem_definition.py:440-447) with the 19-point
-// normal Laplacian of fd_stencils.py:77-103.  Edge ghosts are used here, so
-// the x-then-y-then-z composition of the ghost rules matters.
-// ---------------------------------------------------------------------------
-template <typename T>
-struct AcCoef {
-  T s18;       // 18/eps
-  T eps;       // eps
-  T curv;      // curvature
-  T one_m_curv;// 1-curvature
-  T gab, M, force;
-  T s3;        // 3/eps
-};
-
 template <typename T, int W>
 __device__ __forceinline__ T normal_lap_at(const T (*Pm)[W], const T (*P0)[W], const T (*Pp)[W], int a,
                                            int b, const Geo<T>& g) {
@@ -178,68 +41,10 @@ __device__ __forceinline__ T normal_lap_at(const T (*Pm)[W], const T (*P0)[W], c
   const T R = Pp[a][b], L = Pm[a][b];
   const T Tp = P0[a + 1][b], Bm = P0[a - 1][b];
   const T F = P0[a][b + 1], K = P0[a][b - 1];
-  const T gx = (T(0.5) * (R - L)) * g.idx;
-  const T gy = (T(0.5) * (Tp - Bm)) * g.idy;
-  const T gz = (T(0.5) * (F - K)) * g.idz;
-  const T t1 = ((gx * gx) * ((R - T(2) * C) + L)) * g.idx2;
-  const T t2 = ((gy * gy) * ((Tp - T(2) * C) + Bm)) * g.idy2;
-  const T t3 = ((gz * gz) * ((F - T(2) * C) + K)) * g.idz2;
   const T cxy = ((Pp[a + 1][b] + Pm[a - 1][b]) - Pm[a + 1][b]) - Pp[a - 1][b];
   const T cxz = ((Pp[a][b + 1] + Pm[a][b - 1]) - Pm[a][b + 1]) - Pp[a][b - 1];
   const T cyz = ((P0[a + 1][b + 1] + P0[a - 1][b - 1]) - P0[a - 1][b + 1]) - P0[a + 1][b - 1];
-  const T t4 = ((((T(0.5) * gx) * gy) * cxy) * g.idx) * g.idy;
-  const T t5 = ((((T(0.5) * gx) * gz) * cxz) * g.idx) * g.idz;
-  const T t6 = ((((T(0.5) * gy) * gz) * cyz) * g.idy) * g.idz;
-  const T num = ((((t1 + t2) + t3) + t4) + t5) + t6;
-  T n2 = ((gx * gx) + (gy * gy)) + (gz * gz);
-  if (n2 <= static_cast<T>(1e-7)) n2 = T(1);
-  return num / n2;
-}
-
-template <typename T>
-__global__ __launch_bounds__(NT) void ac_rhs_kernel(const T* __restrict__ u, T* __restrict__ out, Dims d, Bc bc,
-                                                    Geo<T> g, AcCoef<T> k, Epi ep, TileGrid tg) {
-  constexpr int PY = TileCfg<T>::PY, BY = NTY * PY;
-  constexpr int W = BZ + 2, ROWS = BY + 2, NR = 4;
-  __shared__ T cs[NR][ROWS][W];
-  const int tz = threadIdx.x, ty = threadIdx.y, tid = ty * BZ + tz;
-  const TileOrigin o = tile_origin<BY>(tg, d, xcd_tile(blockIdx.x, gridDim.x));
-  const int64_t z0 = o.z0, y0 = o.y0, x0 = o.x0, x1 = o.x1;
-  const T* uc = u + o.ch * d.vol();
-  T* oc = out + o.ch * d.vol();
-  PlaneLoader<T, 1, ROWS, W, true, true> pl;
-  pl.init(y0, z0, d, bc, tid);
-  for (int64_t xg = x0 - 1; xg <= x0 + 1; ++xg) {
-    pl.fetch(uc, xg, d, bc);
-    pl.commit(&cs[ring<NR>(xg - x0)][0][0], bc, tid);
-  }
-  if (x0 + 2 <= x1) pl.fetch(uc, x0 + 2, d, bc);
-  __syncthreads();
-  const int64_t plane = d.ny * d.nz;
-  const int64_t gz = z0 + tz;
-  for (int64_t x = x0; x < x1; ++x) {
-    if (x + 2 <= x1) pl.commit(&cs[ring<NR>(x + 2 - x0)][0][0], bc, tid);
-    if (x + 3 <= x1) pl.fetch(uc, x + 3, d, bc);
-    const T(*Pm)[W] = cs[ring<NR>(x - 1 - x0)];
-    const T(*P0)[W] = cs[ring<NR>(x - x0)];
-    const T(*Pp)[W] = cs[ring<NR>(x + 1 - x0)];
-#pragma unroll
-    for (int q = 0; q < PY; ++q) {
-      const int yy = ty + NTY * q;
-      const int64_t gy = y0 + yy;
-      if (gy >= d.ny || gz >= d.nz) continue;
-      const int a = yy + 1, b = tz + 1;
-      const T phi = P0[a][b];
-      const T pot = ((k.s18 * phi) * (T(1) - phi)) * (T(1) - T(2) * phi);
-      const T lap = k.curv * lap7(phi, Pp[a][b], Pm[a][b], P0[a + 1][b], P0[a - 1][b], P0[a][b + 1],
-                                  P0[a][b - 1], g);
-      const T nlap = k.one_m_curv * normal_lap_at<T, W>(Pm, P0, Pp, a, b, g);
-      const T df = k.gab * ((lap + nlap) - (pot / T(2)) / k.eps) +
-                   ((k.s3 * phi) * (T(1) - phi)) * k.force;
-      epilogue(ep, uc, oc, x * plane + gy * d.nz + gz, k.M * df);
-    }
-    __syncthreads();
-  }
+  return normal_lap_of(C, R, L, Tp, Bm, F, K, cxy, cxz, cyz, g);
 }
 
 // ---------------------------------------------------------------------------
@@ -703,29 +508,6 @@ dim3 stencil_grid(const Dims& d, TileGrid* tg, int64_t target = XCHUNK_BLOCKS) {
 }
 
 template <typename T>
-int launch_rd(const void* u, void* out, const Dims& d, const Bc& bc, const evx_grid* g, double D,
-              const Epi& ep, hipStream_t s) {
-  TileGrid tg;
-  dim3 grid = stencil_grid<T>(d, &tg, EVX_RESIDENT_ROUND(rd_rhs_kernel<T>));
-  hipLaunchKernelGGL(rd_rhs_kernel<T>, grid, dim3(BZ, NTY), 0, s, static_cast<const T*>(u),
-                     static_cast<T*>(out), d, bc, make_geo<T>(g), static_cast<T>(D), ep, tg);
-  return check_launch("rd_rhs_kernel");
-}
-
-template <typename T>
-int launch_gs(const void* u, void* out, const Dims& d, const Bc& bc, const evx_grid* g, double Da, double Db,
-              double feed, double kill, const Epi& ep, hipStream_t s) {
-  TileGrid tg;
-  Dims d1 = d;
-  d1.c = 1;  // one block covers both species of its tile
-  dim3 grid = stencil_grid<T>(d1, &tg, EVX_RESIDENT_ROUND(gs_rhs_kernel<T>));
-  GsCoef<T> k{static_cast<T>(Da), static_cast<T>(Db), static_cast<T>(feed), static_cast<T>(kill)};
-  hipLaunchKernelGGL(gs_rhs_kernel<T>, grid, dim3(BZ, NTY), 0, s, static_cast<const T*>(u),
-                     static_cast<T*>(out), d1, bc, make_geo<T>(g), k, ep, tg);
-  return check_launch("gs_rhs_kernel");
-}
-
-template <typename T>
 int launch_ch(const void* u, void* out, const Dims& d, const Bc& bc, const evx_grid* g, double eps,
               double D, const Epi& ep, hipStream_t s) {
   TileGrid tg;
@@ -769,19 +551,6 @@ int launch_ch_periodic(const T* u, T* out, const Dims& d, const Geo<T>& g, const
   return check_launch("ch_periodic_kernel");
 }
 
-template <typename T>
-int launch_ac(const void* u, void* out, const Dims& d, const Bc& bc, const evx_grid* g, double eps,
-              double gab, double M, double force, double curv, const Epi& ep, hipStream_t s) {
-  TileGrid tg;
-  dim3 grid = stencil_grid<T>(d, &tg, EVX_RESIDENT_ROUND(ac_rhs_kernel<T>));
-  AcCoef<T> k{static_cast<T>(18.0 / eps), static_cast<T>(eps), static_cast<T>(curv),
-              static_cast<T>(1.0 - curv), static_cast<T>(gab), static_cast<T>(M),
-              static_cast<T>(force), static_cast<T>(3.0 / eps)};
-  hipLaunchKernelGGL(ac_rhs_kernel<T>, grid, dim3(BZ, NTY), 0, s, static_cast<const T*>(u),
-                     static_cast<T*>(out), d, bc, make_geo<T>(g), k, ep, tg);
-  return check_launch("ac_rhs_kernel");
-}
-
 inline unsigned flat_blocks(int64_t n) {
   int64_t b = (n + 255) / 256;
   if (b > 65535LL * 16) b = 65535LL * 16;
@@ -822,8 +591,7 @@ int stencil_rhs_rd_periodic(int32_t dtype, const void* u, void* out, const Dims&
   evx_grid g{d.c, d.nx, d.ny, d.nz, {0.0, 0.0, 0.0}, {div_dx2[0], div_dx2[1], div_dx2[2]}};
   Bc b{};
   const Epi ep{EVX_OUT_RHS, 0.0, nullptr, nullptr, nullptr};
-  return dtype == EVX_F32 ? launch_rd<float>(u, out, d, b, &g, D, ep, s)
-                          : launch_rd<double>(u, out, d, b, &g, D, ep, s);
+  return launch_rd(dtype, u, out, d, b, &g, D, ep, s);
 }
 }  // namespace evx
 
@@ -881,8 +649,7 @@ extern "C" int evx_rd_rhs(int32_t dtype, const void* u, void* out, const evx_gri
   EVX_TRY(check_common(dtype, u, out, g, bc, &d, &b));
   EVX_TRY(check_epi(e, u, out, &ep));
   hipStream_t s = static_cast<hipStream_t>(stream);
-  return dtype == EVX_F32 ? launch_rd<float>(u, out, d, b, g, D, ep, s)
-                          : launch_rd<double>(u, out, d, b, g, D, ep, s);
+  return launch_rd(dtype, u, out, d, b, g, D, ep, s);
 }
 
 extern "C" int evx_coupled_rd_rhs(int32_t dtype, const void* u, void* out, const evx_grid* g, const evx_bc* bc,
@@ -896,8 +663,7 @@ extern "C" int evx_coupled_rd_rhs(int32_t dtype, const void* u, void* out, const
   EVX_TRY(check_epi(e, u, out, &ep));
   if (d.c != 2) return fail(EVX_ERR_INVALID, "the two-species right-hand side needs exactly two channels");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  return dtype == EVX_F32 ? launch_gs<float>(u, out, d, b, g, D_A, D_B, feed, kill, ep, s)
-                          : launch_gs<double>(u, out, d, b, g, D_A, D_B, feed, kill, ep, s);
+  return launch_gs(dtype, u, out, d, b, g, D_A, D_B, feed, kill, ep, s);
 }
 
 extern "C" int evx_ch_rhs(int32_t dtype, const void* u, void* out, const evx_grid* g, const evx_bc* bc,
@@ -927,8 +693,7 @@ extern "C" int evx_ac_rhs(int32_t dtype, const void* u, void* out, const evx_gri
   EVX_TRY(check_epi(e, u, out, &ep));
   if (!(eps != 0.0)) return fail(EVX_ERR_INVALID, "eps must be nonzero");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  return dtype == EVX_F32 ? launch_ac<float>(u, out, d, b, g, eps, gab, M, force, curvature, ep, s)
-                          : launch_ac<double>(u, out, d, b, g, eps, gab, M, force, curvature, ep, s);
+  return launch_ac(dtype, u, out, d, b, g, eps, gab, M, force, curvature, ep, s);
 }
 
 extern "C" int evx_simplex_project(int32_t dtype, const void* phis, void* out, int32_t n_phases, int64_t voxels,

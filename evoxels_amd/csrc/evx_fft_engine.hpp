@@ -1,4 +1,4 @@
-// Device-side FFT building blocks: radix-2/3/4/5/8 butterflies and a
+// Device-side FFT building blocks: butterflies of radix 2 to 16 and a
 // compile-time mixed-radix Stockham engine that keeps each thread's values in
 // registers between passes.
 //
@@ -89,6 +89,123 @@ __device__ __forceinline__ void dft_fixed(cpx<T>* x) {
   else dft8<T, INV>(x);
 }
 
+// Good-Thomas factorisation of a butterfly of A*B points, A and B coprime:
+// no twiddles between the two stages.
+template <int A, int B>
+constexpr int crt(int a, int b) {
+  for (int k = 0; k < A * B; ++k)
+    if (k % A == a && k % B == b) return k;
+  return 0;
+}
+
+template <typename T, bool INV, int R>
+__device__ __forceinline__ void dft_any(cpx<T>* x);
+
+template <typename T, bool INV, int A, int B>
+__device__ __forceinline__ void dft_coprime(cpx<T>* x) {
+  constexpr int N = A * B;
+  cpx<T> t[B][A];
+#pragma unroll
+  for (int j = 0; j < B; ++j) {
+#pragma unroll
+    for (int i = 0; i < A; ++i) t[j][i] = x[(B * i + A * j) % N];
+    dft_any<T, INV, A>(t[j]);
+  }
+#pragma unroll
+  for (int i = 0; i < A; ++i) {
+    cpx<T> y[B];
+#pragma unroll
+    for (int j = 0; j < B; ++j) y[j] = t[j][i];
+    dft_any<T, INV, B>(y);
+#pragma unroll
+    for (int j = 0; j < B; ++j) x[crt<A, B>(i, j)] = y[j];
+  }
+}
+
+// Butterfly of A*A points (9, 16): two stages of radix A with the inner
+// twiddles w_{A*A}^(i*j) as constants.
+template <typename T, bool INV, int A>
+__device__ __forceinline__ void dft_square(cpx<T>* x) {
+  constexpr T C9[5] = {T(1), T(0.76604444311897803520), T(0.17364817766693034885), T(-0.5),
+                       T(-0.93969262078590838405)};
+  constexpr T S9[5] = {T(0), T(0.64278760968653932632), T(0.98480775301220805937), T(0.86602540378443864676),
+                       T(0.34202014332566873304)};
+  constexpr T C16[10] = {T(1), T(0.92387953251128675613), T(0.70710678118654752440), T(0.38268343236508977173), T(0),
+                         T(-0.38268343236508977173), T(-0.70710678118654752440), T(-0.92387953251128675613), T(-1),
+                         T(-0.92387953251128675613)};
+  constexpr T S16[10] = {T(0), T(0.38268343236508977173), T(0.70710678118654752440), T(0.92387953251128675613), T(1),
+                         T(0.92387953251128675613), T(0.70710678118654752440), T(0.38268343236508977173), T(0),
+                         T(-0.38268343236508977173)};
+  cpx<T> t[A][A];
+#pragma unroll
+  for (int j = 0; j < A; ++j) {  // j = n mod A
+#pragma unroll
+    for (int i = 0; i < A; ++i) t[j][i] = x[A * i + j];
+    dft_any<T, INV, A>(t[j]);
+#pragma unroll
+    for (int i = 1; i < A; ++i) {
+      if (j == 0) continue;
+      const cpx<T> w = A == 3 ? cpx<T>{C9[i * j], -S9[i * j]} : cpx<T>{C16[i * j], -S16[i * j]};
+      if (A == 4 && i * j == 4) t[j][i] = mul_mi<T, INV>(t[j][i]);
+      else t[j][i] = INV ? cmulc(t[j][i], w) : cmul(t[j][i], w);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < A; ++i) {
+    cpx<T> y[A];
+#pragma unroll
+    for (int j = 0; j < A; ++j) y[j] = t[j][i];
+    dft_any<T, INV, A>(y);
+#pragma unroll
+    for (int j = 0; j < A; ++j) x[i + A * j] = y[j];
+  }
+}
+
+template <typename T, bool INV>
+__device__ __forceinline__ void dft7(cpx<T>* x) {
+  constexpr T c[4] = {T(1), T(0.62348980185873353053), T(-0.22252093395631440429), T(-0.90096886790241912624)};
+  constexpr T s[4] = {T(0), T(0.78183148246802980871), T(0.97492791218182360702), T(0.43388373911755812048)};
+  cpx<T> a[4], b[4];
+  cpx<T> y0 = x[0];
+#pragma unroll
+  for (int r = 1; r <= 3; ++r) {
+    a[r] = cadd(x[r], x[7 - r]);
+    b[r] = csub(x[r], x[7 - r]);
+    y0 = cadd(y0, a[r]);
+  }
+  const cpx<T> x0 = x[0];
+  x[0] = y0;
+#pragma unroll
+  for (int q = 1; q <= 3; ++q) {
+    cpx<T> u = x0, v = {T(0), T(0)};
+#pragma unroll
+    for (int r = 1; r <= 3; ++r) {
+      const int e = (q * r) % 7;
+      const T cc = c[e <= 3 ? e : 7 - e], ss = e <= 3 ? s[e] : -s[7 - e];
+      u.x += cc * a[r].x;
+      u.y += cc * a[r].y;
+      v.x += ss * b[r].x;
+      v.y += ss * b[r].y;
+    }
+    v = mul_mi<T, INV>(v);
+    x[q] = cadd(u, v);
+    x[7 - q] = csub(u, v);
+  }
+}
+
+template <typename T, bool INV, int R>
+__device__ __forceinline__ void dft_any(cpx<T>* x) {
+  if constexpr (R == 1) return;
+  else if constexpr (R == 6) dft_coprime<T, INV, 2, 3>(x);
+  else if constexpr (R == 7) dft7<T, INV>(x);
+  else if constexpr (R == 9) dft_square<T, INV, 3>(x);
+  else if constexpr (R == 10) dft_coprime<T, INV, 2, 5>(x);
+  else if constexpr (R == 12) dft_coprime<T, INV, 4, 3>(x);
+  else if constexpr (R == 15) dft_coprime<T, INV, 3, 5>(x);
+  else if constexpr (R == 16) dft_square<T, INV, 4>(x);
+  else dft_fixed<T, INV, R>(x);
+}
+
 // --------------------------------------------------------------------------
 // Compile-time engine.  Lay::at(e) returns the LDS slot of element e of the
 // calling thread's line; the engine writes pass outputs there, synchronises,
@@ -140,7 +257,7 @@ __device__ __forceinline__ void stockham(cpx<T> (&v)[N / TPL], const Lay& lay, i
         x[r] = INV ? cmulc(x[r], w) : cmul(x[r], w);
       }
     }
-    dft_fixed<T, INV, R>(x);
+    dft_any<T, INV, R>(x);
 #pragma unroll
     for (int r = 0; r < R; ++r) y[s][r] = x[r];
   }

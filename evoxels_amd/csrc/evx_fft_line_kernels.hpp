@@ -6,124 +6,6 @@
 
 namespace evx {
 
-// ------------------------------------------------------------ butterflies --
-// Good-Thomas factorisation of a butterfly of A*B points, A and B coprime:
-// no twiddles between the two stages.
-template <int A, int B>
-constexpr int crt(int a, int b) {
-  for (int k = 0; k < A * B; ++k)
-    if (k % A == a && k % B == b) return k;
-  return 0;
-}
-
-template <typename T, bool INV, int R>
-__device__ __forceinline__ void dft_any(cpx<T>* x);
-
-template <typename T, bool INV, int A, int B>
-__device__ __forceinline__ void dft_coprime(cpx<T>* x) {
-  constexpr int N = A * B;
-  cpx<T> t[B][A];
-#pragma unroll
-  for (int j = 0; j < B; ++j) {
-#pragma unroll
-    for (int i = 0; i < A; ++i) t[j][i] = x[(B * i + A * j) % N];
-    dft_any<T, INV, A>(t[j]);
-  }
-#pragma unroll
-  for (int i = 0; i < A; ++i) {
-    cpx<T> y[B];
-#pragma unroll
-    for (int j = 0; j < B; ++j) y[j] = t[j][i];
-    dft_any<T, INV, B>(y);
-#pragma unroll
-    for (int j = 0; j < B; ++j) x[crt<A, B>(i, j)] = y[j];
-  }
-}
-
-// Butterfly of A*A points (9, 16): two stages of radix A with the inner
-// twiddles w_{A*A}^(i*j) as constants.
-template <typename T, bool INV, int A>
-__device__ __forceinline__ void dft_square(cpx<T>* x) {
-  constexpr T C9[5] = {T(1), T(0.76604444311897803520), T(0.17364817766693034885), T(-0.5),
-                       T(-0.93969262078590838405)};
-  constexpr T S9[5] = {T(0), T(0.64278760968653932632), T(0.98480775301220805937), T(0.86602540378443864676),
-                       T(0.34202014332566873304)};
-  constexpr T C16[10] = {T(1), T(0.92387953251128675613), T(0.70710678118654752440), T(0.38268343236508977173), T(0),
-                         T(-0.38268343236508977173), T(-0.70710678118654752440), T(-0.92387953251128675613), T(-1),
-                         T(-0.92387953251128675613)};
-  constexpr T S16[10] = {T(0), T(0.38268343236508977173), T(0.70710678118654752440), T(0.92387953251128675613), T(1),
-                         T(0.92387953251128675613), T(0.70710678118654752440), T(0.38268343236508977173), T(0),
-                         T(-0.38268343236508977173)};
-  cpx<T> t[A][A];
-#pragma unroll
-  for (int j = 0; j < A; ++j) {  // j = n mod A
-#pragma unroll
-    for (int i = 0; i < A; ++i) t[j][i] = x[A * i + j];
-    dft_any<T, INV, A>(t[j]);
-#pragma unroll
-    for (int i = 1; i < A; ++i) {
-      if (j == 0) continue;
-      const cpx<T> w = A == 3 ? cpx<T>{C9[i * j], -S9[i * j]} : cpx<T>{C16[i * j], -S16[i * j]};
-      if (A == 4 && i * j == 4) t[j][i] = mul_mi<T, INV>(t[j][i]);
-      else t[j][i] = INV ? cmulc(t[j][i], w) : cmul(t[j][i], w);
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < A; ++i) {
-    cpx<T> y[A];
-#pragma unroll
-    for (int j = 0; j < A; ++j) y[j] = t[j][i];
-    dft_any<T, INV, A>(y);
-#pragma unroll
-    for (int j = 0; j < A; ++j) x[i + A * j] = y[j];
-  }
-}
-
-template <typename T, bool INV>
-__device__ __forceinline__ void dft7(cpx<T>* x) {
-  constexpr T c[4] = {T(1), T(0.62348980185873353053), T(-0.22252093395631440429), T(-0.90096886790241912624)};
-  constexpr T s[4] = {T(0), T(0.78183148246802980871), T(0.97492791218182360702), T(0.43388373911755812048)};
-  cpx<T> a[4], b[4];
-  cpx<T> y0 = x[0];
-#pragma unroll
-  for (int r = 1; r <= 3; ++r) {
-    a[r] = cadd(x[r], x[7 - r]);
-    b[r] = csub(x[r], x[7 - r]);
-    y0 = cadd(y0, a[r]);
-  }
-  const cpx<T> x0 = x[0];
-  x[0] = y0;
-#pragma unroll
-  for (int q = 1; q <= 3; ++q) {
-    cpx<T> u = x0, v = {T(0), T(0)};
-#pragma unroll
-    for (int r = 1; r <= 3; ++r) {
-      const int e = (q * r) % 7;
-      const T cc = c[e <= 3 ? e : 7 - e], ss = e <= 3 ? s[e] : -s[7 - e];
-      u.x += cc * a[r].x;
-      u.y += cc * a[r].y;
-      v.x += ss * b[r].x;
-      v.y += ss * b[r].y;
-    }
-    v = mul_mi<T, INV>(v);
-    x[q] = cadd(u, v);
-    x[7 - q] = csub(u, v);
-  }
-}
-
-template <typename T, bool INV, int R>
-__device__ __forceinline__ void dft_any(cpx<T>* x) {
-  if constexpr (R == 1) return;
-  else if constexpr (R == 6) dft_coprime<T, INV, 2, 3>(x);
-  else if constexpr (R == 7) dft7<T, INV>(x);
-  else if constexpr (R == 9) dft_square<T, INV, 3>(x);
-  else if constexpr (R == 10) dft_coprime<T, INV, 2, 5>(x);
-  else if constexpr (R == 12) dft_coprime<T, INV, 4, 3>(x);
-  else if constexpr (R == 15) dft_coprime<T, INV, 3, 5>(x);
-  else if constexpr (R == 16) dft_square<T, INV, 4>(x);
-  else dft_fixed<T, INV, R>(x);
-}
-
 // ------------------------------------------------------------------ passes --
 // Line accessors: element e = i + rm of the thread's line, rm block-uniform.
 template <typename T>
@@ -307,13 +189,19 @@ __device__ __forceinline__ void line_pass_r(const LinePass ps, int tl, int tpl, 
 // Prime radix R > 10 through a_r = x_r + x_{R-r}, b_r = x_r - x_{R-r}: outputs
 // q and R - q share sum_r a_r cos(2 pi rq/R) and sum_r b_r sin(2 pi rq/R).  The
 // outputs are formed one pair at a time (a loop, not unrolled) with the
-// coefficients read from the table at a block-uniform index.
+// coefficients read from the table.  The pass has few butterflies (n/R of a
+// line's tpl threads), so the threads left over share their output pairs:
+// thread tl takes butterfly tl mod m and every parts-th pair.  One serial chain
+// of R(R-1)/2 products a butterfly bounded the sweep: a float64 step of
+// 40 x 33 x 31 took 54.8 us with one thread a butterfly and takes 34.5, one of
+// 69 x 92 x 115 110.7 and 93 (MI355X).
 template <typename T, bool INV, int R, typename Src, typename Dst>
 __device__ __forceinline__ void line_pass_prime(const LinePass ps, int tl, int tpl, bool active, const cpx<T>* tw,
                                                 const Src& src, const Dst& dst) {
   constexpr int H = (R - 1) / 2;
-  const int m = ps.m, p = ps.p, i = tl;
-  const bool mine = active && i < m;
+  const int m = ps.m, p = ps.p;
+  const int parts = tpl / m, part = tl / m, i = tl - part * m;
+  const bool mine = active && part < parts;
   __syncthreads();  // the source lines, or in a first pass the table
   cpx<T> x[R];
   if (mine) {
@@ -343,15 +231,16 @@ __device__ __forceinline__ void line_pass_prime(const LinePass ps, int tl, int t
     cpx<T> b0, b1;  // base values of the next output pair
     if constexpr (Dst::BASE) {
       const cpx<T> bs = dst.load_base(j, 0);
-      b0 = dst.load_base(j, p);
-      b1 = dst.load_base(j, (R - 1) * p);
-      dst.store(j, 0, sum, bs);
+      const int q0 = part < H ? part + 1 : H;
+      b0 = dst.load_base(j, q0 * p);
+      b1 = dst.load_base(j, (R - q0) * p);
+      if (part == 0) dst.store(j, 0, sum, bs);
     } else {
-      dst.store(j, 0, sum);
+      if (part == 0) dst.store(j, 0, sum);
     }
     const cpx<T>* const rt = tw + ps.rt;
 #pragma unroll 1
-    for (int q = 1; q <= H; ++q) {
+    for (int q = part + 1; q <= H; q += parts) {
       cpx<T> u = x[0], v = {T(0), T(0)};
       int e = 0;
 #pragma unroll
@@ -367,7 +256,7 @@ __device__ __forceinline__ void line_pass_prime(const LinePass ps, int tl, int t
       v = mul_mi<T, INV>(v);
       if constexpr (Dst::BASE) {
         const cpx<T> c0 = b0, c1 = b1;
-        const int qn = q < H ? q + 1 : q;
+        const int qn = q + parts <= H ? q + parts : q;
         b0 = dst.load_base(j, qn * p);
         b1 = dst.load_base(j, (R - qn) * p);
         dst.store(j, q * p, cadd(u, v), c0);

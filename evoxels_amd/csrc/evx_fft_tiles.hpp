@@ -259,13 +259,16 @@ template <int N> struct FftSpec;
 template <> struct FftSpec<8>    { using R = Rad<8>;          static constexpr int L = 8; };
 template <> struct FftSpec<16>   { using R = Rad<4, 4>;       static constexpr int L = 4; };
 template <> struct FftSpec<32>   { using R = Rad<4, 8>;       static constexpr int L = 8; };
-template <> struct FftSpec<48>   { using R = Rad<3, 4, 4>;    static constexpr int L = 12; };
+template <> struct FftSpec<48>   { using R = Rad<12, 4>;      static constexpr int L = 12; };
 template <> struct FftSpec<64>   { using R = Rad<8, 8>;       static constexpr int L = 8; };
-template <> struct FftSpec<96>   { using R = Rad<3, 4, 4, 2>; static constexpr int L = 12; };
-// 100 = 2*5*2*5: ten values per thread (Rad<4, 5, 5> needs twenty), so a
-// 100^3 grid's sweeps run twice the threads and blocks; the 100^3 float64
-// CH step took 0.0581 instead of 0.0709 ms (MI355X).
-template <> struct FftSpec<100>  { using R = Rad<2, 5, 2, 5>; static constexpr int L = 10; };
+// 48 and 96 at twelve values per thread: one exchange fewer than Rad<3, 4, 4>
+// and Rad<3, 4, 4, 2>; six sweeps of 96^3 float32 40.7 instead of 43 us and
+// 4 x 96^3 float64 91.1 instead of 97.8 us (MI355X).
+template <> struct FftSpec<96>   { using R = Rad<6, 4, 4>;    static constexpr int L = 12; };
+// 100 = 10*10: ten values per thread (Rad<4, 5, 5> needs twenty), one exchange
+// where Rad<2, 5, 2, 5> has three; six sweeps of a 100^3 float64 CH step 50.7
+// instead of 56.8 us (MI355X).
+template <> struct FftSpec<100>  { using R = Rad<10, 10>;     static constexpr int L = 10; };
 // 128 = 2*4*4*4: four values per thread instead of eight (Rad<2, 8, 8>):
 // the 16 x 128^3 inversion gradient 0.3256 -> 0.3187 s, the 48-grid batched
 // step 0.2655 -> 0.2649 ms (MI355X).  The same change for 32 and 64

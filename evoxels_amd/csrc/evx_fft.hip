@@ -24,6 +24,7 @@
 #include "evx_common.hpp"
 #include "evx_fft_engine.hpp"
 #include "evx_fft_lines.hpp"
+#include "evx_fft_planes.hpp"
 #include "evx_fft_tiles.hpp"
 #include "evx_rz_tile.hpp"
 
@@ -219,6 +220,7 @@ struct evx_fft_plan {
   bool fused_rhs = true;       // CH steps: fused right-hand side + z R2C where it applies
   bool step_sums = true;       // one-channel steps: mass and NaN/Inf records from the z C2R epilogue
   const void* sums_ws = nullptr;  // workspace holding the records of the last recording step
+  int64_t sums_n = 0;             // their count
 };
 
 namespace evx {
@@ -380,7 +382,13 @@ int64_t rec_blocks(const evx_fft_plan* p) {
   if (p->d.c != 1) return 0;
   return p->dtype == EVX_F32 ? rec_blocks_t<float>(p) : rec_blocks_t<double>(p);
 }
-size_t rec_bytes(const evx_fft_plan* p) { return align_up((size_t)rec_blocks(p) * sizeof(SumRec)); }
+// Whether a step's z and y sweeps run plane by plane.
+bool use_planes(const evx_fft_plan* p) { return p->fast && plane_sweeps_apply(p->d); }
+// Room for the records of either form: one per z tile or one per plane.
+size_t rec_bytes(const evx_fft_plan* p) {
+  const int64_t n = rec_blocks(p);
+  return align_up((size_t)(n == 0 ? 0 : std::max(n, p->d.nx)) * sizeof(SumRec));
+}
 // Bytes of the forward workspace: right-hand-side staging, spectrum, records.
 size_t fwd_ws_bytes(const evx_fft_plan* p) { return real_bytes(p) + spec_bytes(p) + rec_bytes(p); }
 // Records of a step on workspace ws, or nullptr when this step keeps none.
@@ -430,7 +438,7 @@ int run_x_multiplier(evx_fft_plan* p, void* spec, const Prefac& pf, int64_t pt, 
 
 // Launch trace (armed by evx_fft_plan_trace_next_step).  Kernel kinds:
 enum { TK_RHS = 0, TK_Z_R2C = 1, TK_Y_FWD = 2, TK_X = 3, TK_Y_INV = 4, TK_Z_C2R = 5, TK_RHS_Z_R2C = 6,
-       TK_OTHER = 7 };
+       TK_OTHER = 7, TK_ZY = 8, TK_YZ = 9 };
 
 int trace_start(evx_fft_plan* p, hipStream_t s) {
   p->tpos = 0;
@@ -457,24 +465,51 @@ void trace_end(evx_fft_plan* p) {
   p->tpos = 0;
 }
 
+// z R2C and forward y (inverse y and z C2R) of the planes [a, b), numbered over
+// channels and x, one block per plane.
+template <typename T>
+int run_plane_fwd(evx_fft_plan* p, const void* x, void* spec, int64_t a, int64_t b, hipStream_t s) {
+  return plane_run_fwd<T>(p->ax[2].n, p->ax[2].tw, static_cast<const T*>(x) + a * p->d.plane(),
+                          static_cast<cpx<T>*>(spec) + a * p->d.ny * p->nh, b - a, s);
+}
+template <typename T>
+int run_plane_inv(evx_fft_plan* p, const void* spec, void* out, const void* base, double scale, int64_t a, int64_t b,
+                  SumRec* rec, hipStream_t s) {
+  const int64_t off = a * p->d.plane();
+  return plane_run_inv<T>(p->ax[2].n, p->ax[2].tw, static_cast<const cpx<T>*>(spec) + a * p->d.ny * p->nh,
+                          static_cast<T*>(out) + off, base ? static_cast<const T*>(base) + off : nullptr, scale, b - a,
+                          rec, s);
+}
+
 // rhs == nullptr: the z half spectrum of the right-hand side is already in
 // spec (the fused first sweep).
 template <typename T>
 int spectral_update(evx_fft_plan* p, const void* rhs, void* spec, const void* u, void* u_out, const Prefac& pf,
                     hipStream_t s, SumRec* rec = nullptr) {
-  const int64_t pt = p->pitch;
-  if (rhs) {
-    EVX_TRY(run_z_r2c<T>(p, rhs, spec, pt, s));
-    EVX_TRY(trace_tick(p, TK_Z_R2C, s));
+  const int64_t pt = p->pitch, np = p->d.c * p->d.nx;
+  const bool planes = rhs && use_planes(p);
+  if (planes) {
+    EVX_TRY(run_plane_fwd<T>(p, rhs, spec, 0, np, s));
+    EVX_TRY(trace_tick(p, TK_ZY, s));
+  } else {
+    if (rhs) {
+      EVX_TRY(run_z_r2c<T>(p, rhs, spec, pt, s));
+      EVX_TRY(trace_tick(p, TK_Z_R2C, s));
+    }
+    EVX_TRY((run_strided<T, 0>(p, 1, spec, pf, pt, s)));
+    EVX_TRY(trace_tick(p, TK_Y_FWD, s));
   }
-  EVX_TRY((run_strided<T, 0>(p, 1, spec, pf, pt, s)));
-  EVX_TRY(trace_tick(p, TK_Y_FWD, s));
   EVX_TRY(run_x_multiplier<T>(p, spec, pf, pt, s));
   EVX_TRY(trace_tick(p, TK_X, s));
-  EVX_TRY((run_strided<T, 1>(p, 1, spec, pf, pt, s)));
-  EVX_TRY(trace_tick(p, TK_Y_INV, s));
-  EVX_TRY(run_z_c2r<T>(p, spec, u_out, u, 1.0, pt, s, 0, -1, rec));
-  EVX_TRY(trace_tick(p, TK_Z_C2R, s));
+  if (planes) {
+    EVX_TRY(run_plane_inv<T>(p, spec, u_out, u, 1.0, 0, np, rec, s));
+    EVX_TRY(trace_tick(p, TK_YZ, s));
+  } else {
+    EVX_TRY((run_strided<T, 1>(p, 1, spec, pf, pt, s)));
+    EVX_TRY(trace_tick(p, TK_Y_INV, s));
+    EVX_TRY(run_z_c2r<T>(p, spec, u_out, u, 1.0, pt, s, 0, -1, rec));
+    EVX_TRY(trace_tick(p, TK_Z_C2R, s));
+  }
   trace_end(p);
   return EVX_OK;
 }
@@ -494,11 +529,17 @@ int ch_slab_step(evx_fft_plan* p, const void* u, void* u_out, void* rhs, void* s
   const int64_t xc = stencil_ch_xchunk(p->dtype, d);
   int64_t w = (d.nx + p->slabs - 1) / p->slabs;
   w = (w + xc - 1) / xc * xc;  // slab width: a whole number of CH tile chunks
+  const bool planes = use_planes(p);
   EVX_TRY(trace_start(p, s));
   for (int64_t xa = 0; xa < d.nx; xa += w) {
     const int64_t xb = xa + w < d.nx ? xa + w : d.nx;
     EVX_TRY(stencil_rhs_ch_periodic(p->dtype, u, rhs, d, dd, dd2, prm->eps, prm->D, prm->chan_params, s, xa, xb));
     EVX_TRY(trace_tick(p, TK_RHS, s));
+    if (planes) {
+      EVX_TRY(run_plane_fwd<T>(p, rhs, spec, xa, xb, s));
+      EVX_TRY(trace_tick(p, TK_ZY, s));
+      continue;
+    }
     EVX_TRY(run_z_r2c<T>(p, rhs, spec, pt, s, xa, xb));
     EVX_TRY(trace_tick(p, TK_Z_R2C, s));
     EVX_TRY((run_strided<T, 0>(p, 1, spec, pf, pt, s, xa, xb)));
@@ -508,6 +549,11 @@ int ch_slab_step(evx_fft_plan* p, const void* u, void* u_out, void* rhs, void* s
   EVX_TRY(trace_tick(p, TK_X, s));
   for (int64_t xa = 0; xa < d.nx; xa += w) {
     const int64_t xb = xa + w < d.nx ? xa + w : d.nx;
+    if (planes) {
+      EVX_TRY(run_plane_inv<T>(p, spec, u_out, u, 1.0, xa, xb, nullptr, s));
+      EVX_TRY(trace_tick(p, TK_YZ, s));
+      continue;
+    }
     EVX_TRY((run_strided<T, 1>(p, 1, spec, pf, pt, s, xa, xb)));
     EVX_TRY(trace_tick(p, TK_Y_INV, s));
     EVX_TRY(run_z_c2r<T>(p, spec, u_out, u, 1.0, pt, s, xa, xb));
@@ -713,7 +759,8 @@ int ch_spectral_step(evx_fft_plan* p, const void* u, void* u_out, void* ws, cons
   SumRec* rec = step_recs(p, ws);
   p->sums_ws = nullptr;
   EVX_TRY(trace_start(p, s));
-  if (rz_applies(p, u)) {
+  const bool fused = rz_applies(p, u);
+  if (fused) {
     EVX_TRY(run_rz(p, u, spec, dd, dd2, prm, s));
     EVX_TRY(trace_tick(p, TK_RHS_Z_R2C, s));
     EVX_TRY(spectral_update<float>(p, nullptr, spec, u, u_out, pf, s, rec));
@@ -723,7 +770,10 @@ int ch_spectral_step(evx_fft_plan* p, const void* u, void* u_out, void* ws, cons
     EVX_TRY(p->dtype == EVX_F32 ? spectral_update<float>(p, rhs, spec, u, u_out, pf, s, rec)
                                 : spectral_update<double>(p, rhs, spec, u, u_out, pf, s, rec));
   }
-  if (rec) p->sums_ws = ws;
+  if (rec) {
+    p->sums_ws = ws;
+    p->sums_n = use_planes(p) && !fused ? p->d.nx : rec_blocks(p);
+  }
   return EVX_OK;
 }
 
@@ -742,11 +792,15 @@ int rd_spectral_step(evx_fft_plan* p, const void* u, void* u_out, void* ws, cons
   Prefac pf = make_prefac(p, 0, (-prm->D) * prm->A, prm->dt, prm->spacing);
   pf.etd = etd;
   if (etd) pf.exact = 0;
+  const bool fused = false;
   SumRec* rec = step_recs(p, ws);
   p->sums_ws = nullptr;
   EVX_TRY(p->dtype == EVX_F32 ? spectral_update<float>(p, rhs, spec, u, u_out, pf, s, rec)
                               : spectral_update<double>(p, rhs, spec, u, u_out, pf, s, rec));
-  if (rec) p->sums_ws = ws;
+  if (rec) {
+    p->sums_ws = ws;
+    p->sums_n = use_planes(p) && !fused ? p->d.nx : rec_blocks(p);
+  }
   return EVX_OK;
 }
 
@@ -964,7 +1018,7 @@ extern "C" int evx_fft_plan_step_sums(evx_fft_plan* p, const void* ws, double* o
     return fail(EVX_ERR_INVALID, "no step records on this workspace: the last semi-implicit step of this plan "
                                  "on it kept none (multi-channel, slab or mirrored steps, step sums off)");
   const SumRec* rec = reinterpret_cast<const SumRec*>(static_cast<const char*>(ws) + real_bytes(p) + spec_bytes(p));
-  hipLaunchKernelGGL(fold_recs, dim3(1), dim3(256), 0, static_cast<hipStream_t>(stream), rec, rec_blocks(p), out,
+  hipLaunchKernelGGL(fold_recs, dim3(1), dim3(256), 0, static_cast<hipStream_t>(stream), rec, p->sums_n, out,
                      nonfinite);
   return check_launch("fold_recs");
 }

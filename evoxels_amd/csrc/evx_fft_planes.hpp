@@ -1,0 +1,30 @@
+// Whole-plane sweeps (evx_fft_planes.hip): z R2C and forward y, or inverse y and
+// z C2R, of an x-plane of N x N points in one block, with the half-spectrum plane in
+// LDS, so that the spectrum crosses memory once instead of three times.
+#pragma once
+#include "evx_common.hpp"
+#include "evx_sum.hpp"
+
+namespace evx {
+
+// Whether the steps of a grid run their z and y sweeps plane by plane: ny = nz,
+// one of the lengths whose plane fits LDS in both types (128 takes 143 of
+// 160 KB in float64) and whose N/2 line pairs give a block a plane's work in
+// one round of threads.  Separate sweeps against planes, the semi-implicit
+// step (MI355X, microseconds): 32^3 float32 27.2 / 19.6, 8 x 48^3 float64
+// 45.4 / 28.5, 96^3 float32 40.7 / 31.7, 100^3 float64 50.7 / 42.4,
+// 128^3 float32 50.9 / 42.2, 4 x 128^3 float64 163.4 / 139.2, 16 x 128^3
+// float32 368.5 / 286.7.  8 and 16 keep separate sweeps: a plane of them
+// leaves most of a block idle.
+bool plane_sweeps_apply(const Dims& d);
+
+// Planes 0 .. nplanes-1 of N x N points; twg: the N roots of unity.  With rec, the
+// inverse writes rec[plane]: the compensated float64 sum of its outputs and
+// their NaN / Inf flags.
+template <typename T>
+int plane_run_fwd(int n, const void* twg, const T* x, cpx<T>* spec, int64_t nplanes, hipStream_t s);
+template <typename T>
+int plane_run_inv(int n, const void* twg, const cpx<T>* spec, T* out, const T* base, double scale, int64_t nplanes,
+                  SumRec* rec, hipStream_t s);
+
+}  // namespace evx

@@ -178,19 +178,27 @@ __device__ __forceinline__ void run_sweep(const BArgs& a, int4 it, int tid, unsi
   }
 }
 
-// One sweep of every grid.  A kernel per sweep: each holds only its own
-// sweep's registers and LDS (one kernel for all six needed 97 registers and
-// 27 KB in every launch).
 template <int ST>
 constexpr size_t stage_lds() {
   constexpr size_t z = cmax(cmax(cmax(ZTile<T, 16>::LDS_BYTES, ZTile<T, 32>::LDS_BYTES), cmax(ZTile<T, 48>::LDS_BYTES, ZTile<T, 64>::LDS_BYTES)), cmax(ZTile<T, 96>::LDS_BYTES, ZTile<T, 128>::LDS_BYTES));
   return ST == 0 ? ChB::LDS_BYTES : ST == 1 || ST == 5 ? z : BATCH_LDS;
 }
 
+// One sweep of every grid.  A kernel per sweep: each holds only its own
+// sweep's registers and LDS (one kernel for all six needed 97 registers and
+// 27 KB in every launch).
+//
+// The CH tiles share halos and the y and x bricks share 128-byte lines (a brick's
+// 8 to 32 columns start anywhere in one), so neighbouring items go to one XCD
+// and its L2: right-hand side 63.7 -> 45.6 us, y sweeps 46.6 -> 27.9, x 33.9 -> 33.4
+// on 48 mixed grids of 32 to 128 points an edge (MI355X).  Lines along z share
+// nothing, and there a contiguous range per XCD puts the long lines on a few of
+// them (z R2C 29.8 -> 41.1, z C2R 44.9 -> 65.8), so they stay dealt out in turn.
 template <int ST, bool GROUP>
 __global__ __launch_bounds__(BT) void batch_stage(BArgs a) {
   __shared__ __align__(16) unsigned char smem[stage_lds<ST>()];
-  run_sweep<ST, GROUP>(a, a.items[a.first[ST] + (int)blockIdx.x], threadIdx.x, smem);
+  const unsigned i = ST == 1 || ST == 5 ? blockIdx.x : xcd_tile(blockIdx.x, gridDim.x);
+  run_sweep<ST, GROUP>(a, a.items[a.first[ST] + (int)i], threadIdx.x, smem);
 }
 
 // The whole step in one cooperative launch (all blocks resident): block b

@@ -171,6 +171,9 @@ def call(name: str, *args) -> None:
 
 def stream_handle(device=None) -> C.c_void_p:
     """hipStream_t of torch's current stream on ``device``."""
+    if isinstance(device, torch.device) and device.index is not None:
+        # the handle without a Stream object: 0.2 instead of 2 us a launch
+        return C.c_void_p(torch._C._cuda_getCurrentRawStream(device.index))
     return C.c_void_p(torch.cuda.current_stream(device).cuda_stream)
 
 

@@ -106,7 +106,7 @@ class ODE(ABC):
 
     @property
     def bc_type(self):
-        return tuple(axis_bc[0] for axis_bc in self.bc)
+        return tuple([axis_bc[0] for axis_bc in self.bc])
 
     def _kernel_bcs(self) -> bool:
         """Whether the fused kernels implement this problem's ghost rules:
@@ -141,10 +141,11 @@ class ODE(ABC):
         if not isinstance(u, torch.Tensor) or u.device.type != "cuda":
             raise ValueError("state must be a torch tensor on the ROCm device")
         # the state of a staggered_x grid excludes the two boundary nodes in x
-        nx = self.vg.shape[0] - (2 if self.vg.convention == "staggered_x" else 0)
-        if u.dim() != 4 or tuple(u.shape[1:]) != (nx,) + tuple(self.vg.shape[1:]):
-            raise ValueError(f"state must have shape (C, {nx}, {self.vg.shape[1]}, "
-                             f"{self.vg.shape[2]}), got {tuple(u.shape)}")
+        shape = self.vg.shape
+        nx = shape[0] - (2 if self.vg.convention == "staggered_x" else 0)
+        got = u.shape
+        if len(got) != 4 or got[1] != nx or got[2] != shape[1] or got[3] != shape[2]:
+            raise ValueError(f"state must have shape (C, {nx}, {shape[1]}, {shape[2]}), got {tuple(got)}")
         return u.contiguous()
 
     def _grid(self, u):

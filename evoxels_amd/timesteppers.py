@@ -160,15 +160,14 @@ class PseudoSpectralIMEX(TimeStepper):
     def capturable(self):
         return self._kind is not None
 
-    def _params(self):
+    def _params(self, kind):
         prm = _lib.EvxImexParams()
-        prm.dt = float(self.dt)
-        for a in range(3):
-            prm.spacing[a] = float(self.problem.vg.spacing[a])
         p = self.problem
+        prm.dt = float(self.dt)
+        prm.spacing[:] = [float(v) for v in p.vg.spacing]
         prm.D = float(p.D)
         prm.A = float(p.A)
-        prm.eps = float(p.eps) if "ch" in (self._kind, self._mirror) else 0.0
+        prm.eps = float(p.eps) if kind == "ch" else 0.0
         return prm
 
     def workspace(self, u):
@@ -193,16 +192,18 @@ class PseudoSpectralIMEX(TimeStepper):
 
     def step_into(self, u, out):
         """Fused step writing u + update into ``out`` (``out`` may be ``u``)."""
+        # asked for once: it looks at every closure and boundary of the problem
+        kind = self._kind
         plan, ws = self.workspace(u)
-        prm = self._params()
-        fn = self._FUSED[self._kind]
+        fn = self._FUSED[kind]
+        prm = self._params(kind)
         _lib.call(fn, plan.handle, _lib.ptr(u), _lib.ptr(out), _lib.ptr(ws), C.byref(prm),
                   _lib.stream_handle(u.device))
         return out
 
     _ETD = 0
 
-    def _mirror_step(self, u):
+    def _mirror_step(self, u, kind):
         """Fused step with x non-periodic: the plan covers the mirror-extended
         x length (2n, or 2n+2 on staggered_x grids)."""
         p = self.problem
@@ -213,9 +214,9 @@ class PseudoSpectralIMEX(TimeStepper):
         if self._ws is None or self._ws.numel() < plan.workspace_bytes or self._ws.device != u.device:
             self._ws = torch.empty(plan.workspace_bytes, dtype=torch.uint8, device=u.device)
         out = torch.empty_like(u)
-        prm = self._params()
+        prm = self._params(kind)
         bc = _lib.make_bc(p.bc, p.vg.convention)
-        fn = "evx_ch_imex_step_mirror" if self._mirror == "ch" else "evx_rd_imex_step_mirror"
+        fn = "evx_ch_imex_step_mirror" if kind == "ch" else "evx_rd_imex_step_mirror"
         _lib.call(fn, plan.handle, _lib.ptr(u), _lib.ptr(out), _lib.ptr(self._ws), C.byref(prm), C.byref(bc),
                   int(staggered), self._ETD, _lib.stream_handle(u.device))
         return out
@@ -224,9 +225,10 @@ class PseudoSpectralIMEX(TimeStepper):
         if self._kind is not None:
             u = self.problem._check_state(u)
             return self.step_into(u, torch.empty_like(u))
-        if self._mirror is not None and u.shape[0] == 1 and \
+        kind = self._mirror
+        if kind is not None and u.shape[0] == 1 and \
                 not any(isinstance(v, torch.Tensor) for v in (self.problem.bc[0][1] or ())):
-            return self._mirror_step(self.problem._check_state(u))
+            return self._mirror_step(self.problem._check_state(u), kind)
         vg = self.problem.vg
         dc = self.pad(self.problem.rhs(t, u))
         dc_fft = vg.rfftn(dc, dc.shape)

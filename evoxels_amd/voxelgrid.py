@@ -248,10 +248,11 @@ class VoxelGridHip(FDStencils):
 
     def plan(self, shape4, dtype=None):
         dtype = dtype or self.precision
-        key = (dtype, tuple(int(v) for v in shape4))
-        if key not in self._plans:
-            self._plans[key] = _FFTPlan(_lib.dtype_code(dtype), *key[1])
-        return self._plans[key]
+        key = (dtype, *shape4)
+        plan = self._plans.get(key)
+        if plan is None:
+            plan = self._plans[key] = _FFTPlan(_lib.dtype_code(dtype), *(int(v) for v in shape4))
+        return plan
 
     def reduce_workspace(self, channels):
         lib = _lib.load()

@@ -638,7 +638,7 @@ def configs_leg(cpu):
     ms = _time_steps(lambda: mp.rhs(0.0, ph), 50)
     out["f4_multiphase_ac_rhs_3phases_128cubed_fp32"] = {"ms_per_call": round(ms, 4),
                                                          "voxel_calls_per_s": n ** 3 / (ms * 1e-3),
-                                                         "note": "projection kernel, ghost pad, padded RHS kernel"}
+                                                         "note": "one kernel from the raw phases"}
     x, y, z = np.meshgrid(*[np.arange(n) / n] * 3, indexing="ij")
     sbm = ReactionDiffusionSBM(vg, D=1.0, mask=0.5 + 0.3 * np.cos(4 * np.pi * x) * np.cos(2 * np.pi * y),
                                bc=(("dirichlet", (0.0, 1.0)), "periodic", "periodic"), bc_flux=1.0)

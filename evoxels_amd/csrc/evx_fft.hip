@@ -6,7 +6,8 @@
 // (nh); the steps' workspace spectrum uses pitch = nh.
 //
 // Transforms are mixed-radix Stockham (self-sorting, decimation in time)
-// passes: size-specialised kernels (evx_fft_tiles.hpp) where one exists, the
+// passes: whole-plane z and y sweeps for square y-z planes of some sizes
+// (evx_fft_planes.hip), size-specialised kernels (evx_fft_tiles.hpp) where one exists, the
 // runtime-radix line kernels (evx_fft_lines.hpp) for every other length with
 // prime factors up to 31.
 //
@@ -16,6 +17,7 @@
 //   x : forward C2C along x, times prefac(k)/N, inverse C2C along x
 //   y : inverse C2C along y
 //   z : C2R of line pairs, u_out = u + update
+// With whole-plane sweeps z and y, and y and z, are one sweep each.
 #include <algorithm>
 #include <cmath>
 #include <cstring>

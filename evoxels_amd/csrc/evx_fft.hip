@@ -385,7 +385,7 @@ int64_t rec_blocks(const evx_fft_plan* p) {
   return p->dtype == EVX_F32 ? rec_blocks_t<float>(p) : rec_blocks_t<double>(p);
 }
 // Whether a step's z and y sweeps run plane by plane.
-bool use_planes(const evx_fft_plan* p) { return p->fast && plane_sweeps_apply(p->d); }
+bool use_planes(const evx_fft_plan* p) { return p->fast && plane_sweeps_apply(p->dtype, p->d); }
 // Room for the records of either form: one per z tile or one per plane.
 size_t rec_bytes(const evx_fft_plan* p) {
   const int64_t n = rec_blocks(p);

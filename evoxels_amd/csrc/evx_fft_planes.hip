@@ -215,8 +215,9 @@ __global__ __launch_bounds__((PGeo<T, N>::THREADS)) void plane_inv(const cpx<T>*
 
 }  // namespace
 
-bool plane_sweeps_apply(const Dims& d) {
+bool plane_sweeps_apply(int dtype, const Dims& d) {
   if (d.ny != d.nz) return false;
+  if (dtype == EVX_F64 && d.ny == 128 && d.c * d.nx < 48) return false;
   switch (d.ny) {
 #define X(N) case N:
     EVX_PLANE_SIZES(X)

@@ -15,8 +15,12 @@ namespace evx {
 // 45.4 / 28.5, 96^3 float32 40.7 / 31.7, 100^3 float64 50.7 / 42.4,
 // 128^3 float32 50.9 / 42.2, 4 x 128^3 float64 163.4 / 139.2, 16 x 128^3
 // float32 368.5 / 286.7.  8 and 16 keep separate sweeps: a plane of them
-// leaves most of a block idle.
-bool plane_sweeps_apply(const Dims& d);
+// leaves most of a block idle.  A float64 plane of 128 takes a whole CU and 35 us
+// for both sweeps however few there are, so it needs 48 of them: separate sweeps
+// / planes of n x 128^2 float64 take 28.9 / 33.2 us at n = 16, 33.6 / 34.5 at 32,
+// 38.4 / 35.2 at 64, 52.9 / 38.9 at 128.  The others win from the first plane on
+// (8 x 96^2 float64 36.7 / 26.8, 16 x 128^2 float32 27.7 / 22.6).
+bool plane_sweeps_apply(int dtype, const Dims& d);
 
 // Planes 0 .. nplanes-1 of N x N points; twg: the N roots of unity.  With rec, the
 // inverse writes rec[plane]: the compensated float64 sum of its outputs and

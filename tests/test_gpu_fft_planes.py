@@ -21,8 +21,9 @@ P3 = (("periodic", None),) * 3
 
 
 @pytest.mark.parametrize("precision", ["float32", "float64"])
-@pytest.mark.parametrize("nx,c", [(1, 3), (5, 1), (9, 2)])
-@pytest.mark.parametrize("n", [32, 48, 64, 96, 100, 128])
+@pytest.mark.parametrize("n,nx,c", [(n, nx, c) for n in (32, 48, 64, 96, 100, 128)
+                                    for nx, c in ((1, 3), (5, 1), (9, 2))]
+                         + [(128, 46, 1), (128, 48, 1), (128, 25, 2)])  # 128 in float64: from 48 planes on
 def test_square_planes(n, nx, c, precision):
     shape = (nx, n, n)
     vf = evx.VoxelFields(shape, tuple(s * k for s, k in zip((0.9, 1.1, 1.3), shape)))

@@ -21,7 +21,7 @@ import numpy as np
 import torch
 
 from . import _lib
-from .voxelgrid import VoxelGridHip
+from .voxelgrid import CellCenteredBCs, StaggeredXBCs, VoxelGridHip
 
 try:  # analytic right-hand sides for convergence tests (problem_definition.py:223-224,322-326,408-419)
     import sympy as sp
@@ -52,14 +52,18 @@ class ODE(ABC):
     def initialize_boundary_conditions(self):
         """BC normalisation and validation (problem_definition.py:60-115).  All
         specialised paddings of the reference are one HIP kernel here."""
+        self._pad_bc = self._builtin_pad = self._choose_pad()
+        self._pad_kinds = self.bc_type
+
+    def _choose_pad(self):
+        """Normalises ``bc`` and returns the padding that applies it."""
         bc = getattr(self, "bc", None)
         if bc is None or bc == "fully_periodic":
             self.bc = (("periodic", None), ("periodic", None), ("periodic", None))
             if self.vg.convention == "staggered_x":
                 raise NotImplementedError("a staggered_x grid carries boundary nodes in x; a fully periodic "
                                           "problem belongs on a cell_center grid (boundary_conditions.py:89-94)")
-            self._pad_bc = lambda f: self.vg.bc.pad_bc(f, self.bc)
-            return
+            return lambda f: self.vg.bc.pad_bc(f, self.bc)
         if len(bc) != 3:
             raise ValueError("bc must contain exactly three axis entries ordered as (x, y, z).")
         normalized = []
@@ -93,16 +97,13 @@ class ODE(ABC):
             # the reference's specialised paddings (problem_definition.py:105-115);
             # any other combination reaches StaggeredXBCs.pad_bc, which raises
             if self.bc_type == ("dirichlet", "periodic", "periodic"):
-                self._pad_bc = lambda f: self.vg.bc.pad_dirichlet_periodic(f, self.bc[0][1][0], self.bc[0][1][1])
-            elif self.bc_type == ("neumann", "periodic", "periodic"):
-                self._pad_bc = self.vg.bc.pad_zero_flux_periodic
-            elif self.bc_type == ("periodic", "periodic", "periodic"):
+                return lambda f: self.vg.bc.pad_dirichlet_periodic(f, self.bc[0][1][0], self.bc[0][1][1])
+            if self.bc_type == ("neumann", "periodic", "periodic"):
+                return self.vg.bc.pad_zero_flux_periodic
+            if self.bc_type == ("periodic", "periodic", "periodic"):
                 raise NotImplementedError("a staggered_x grid carries boundary nodes in x; a fully periodic "
                                           "problem belongs on a cell_center grid (boundary_conditions.py:89-94)")
-            else:
-                self._pad_bc = lambda f: self.vg.bc.pad_bc(f, self.bc)
-            return
-        self._pad_bc = lambda f: self.vg.bc.pad_bc(f, self.bc)
+        return lambda f: self.vg.bc.pad_bc(f, self.bc)
 
     @property
     def bc_type(self):
@@ -118,6 +119,21 @@ class ODE(ABC):
             return True
         return self.bc_type == ("dirichlet", "periodic", "periodic") and \
             not any(isinstance(v, torch.Tensor) for v in self.bc[0][1])
+
+    def _own_pad(self) -> bool:
+        """True while the ghost values are the built-in ones: ``pad_bc``, the
+        padding it calls and the grid's boundary rules are all unreplaced.  A
+        kernel that forms ghosts itself must not run when the user's padding
+        is another function (or was chosen for other boundary kinds)."""
+        mine, vg = vars(self), self.vg
+        rules = vg.bc
+        return "pad_bc" not in mine and type(self).pad_bc is ODE.pad_bc and \
+            mine.get("_pad_bc") is not None and mine["_pad_bc"] is mine.get("_builtin_pad") and \
+            (vg.convention == "cell_center" or mine.get("_pad_kinds") == self.bc_type) and \
+            type(rules) in (CellCenteredBCs, StaggeredXBCs) and len(vars(rules)) == 1 and \
+            not {"pad_bc", "pad_staggered_x", "pad_periodic"} & vars(vg).keys() and \
+            type(vg).pad_bc is VoxelGridHip.pad_bc and type(vg).pad_periodic is VoxelGridHip.pad_periodic and \
+            type(vg).pad_staggered_x is VoxelGridHip.pad_staggered_x
 
     # ---- fused-kernel protocol used by the time steppers -----------------
     fused = False
@@ -495,8 +511,8 @@ class MultiPhaseAllenCahn(SemiLinearODE):
 
     def _one_launch(self, u):
         values = [v for _, vals in self.bc if vals is not None for v in vals]
-        return self._kernel_bcs() and not any(isinstance(v, torch.Tensor) for v in values) and \
-            u.shape[2] * u.shape[3] < 2 ** 31
+        return self._own_pad() and self._kernel_bcs() and \
+            not any(isinstance(v, torch.Tensor) for v in values) and u.shape[2] * u.shape[3] < 2 ** 31
 
     def launch(self, u, out, epilogue):
         euclid = getattr(self.project_to_simplex, "__func__", None) is \
@@ -514,7 +530,7 @@ class MultiPhaseAllenCahn(SemiLinearODE):
             out = torch.empty_like(phis)
             self.launch(phis, out, _lib.make_epilogue())
             return out
-        if self._kernel_path(n):  # ghost values given as fields: pad between the kernels
+        if self._kernel_path(n):  # ghost values given as fields or by another padding: pad between the kernels
             dt_code = _lib.dtype_code(phis.dtype)
             stream = _lib.stream_handle(phis.device)
             proj = torch.empty_like(phis)

@@ -214,6 +214,12 @@ def _is_default(fn) -> bool:
     return getattr(fn, "_evx_default", False)
 
 
+def _carries_derivatives(u) -> bool:
+    """Whether ``u`` is part of an autograd graph or holds a forward-mode tangent."""
+    return (u.requires_grad and torch.is_grad_enabled()) or \
+        torch.autograd.forward_ad.unpack_dual(u).tangent is not None
+
+
 @dataclass
 class ReactionDiffusion(SemiLinearODE):
     """problem_definition.py:191-229."""
@@ -504,10 +510,12 @@ class MultiPhaseAllenCahn(SemiLinearODE):
             proj in (MultiPhaseAllenCahn._sloppy_simplex_projection, MultiPhaseAllenCahn._euclidean_simplex_projection)
 
     def fused_for(self, u):
-        """Whether one kernel evaluates the right-hand side of ``u``: up to
-        eight phases, built-in projection and potential, scalar ghost rules."""
+        """Whether one kernel evaluates the step of ``u``: up to eight phases,
+        built-in projection and potential, scalar ghost rules.  A state that
+        carries derivatives takes the composition, whose update is a tensor
+        expression of the state and stays in its graph."""
         return isinstance(u, torch.Tensor) and u.dim() == 4 and self._kernel_path(u.shape[0]) and \
-            self._own_rhs(MultiPhaseAllenCahn) and self._one_launch(u)
+            self._own_rhs(MultiPhaseAllenCahn) and not _carries_derivatives(u) and self._one_launch(u)
 
     def _one_launch(self, u):
         values = [v for _, vals in self.bc if vals is not None for v in vals]

@@ -93,3 +93,22 @@ def test_padding_chosen_for_other_walls_stays():
     p.bc = (("dirichlet", (0.3, 0.8)),) + p.bc[1:]
     got = p.rhs(0.0, u)
     assert float((got - want).abs().max()) < 1e-12 * float(want.abs().max())
+
+
+@pytest.mark.parametrize("stepper", [ForwardEuler, RungeKutta4])
+def test_derivatives_of_the_state_pass_through(stepper):
+    """The right-hand side has no derivative of its own, the update u + dt*r does."""
+    p = MultiPhaseAllenCahn(grid((5, 6, 7)), bc=BC)
+    step = stepper(p, 0.01)
+    u = phases((5, 6, 7))
+    plain = step.step(0.0, u)
+    v = u.clone().requires_grad_()
+    w = torch.rand_like(u)
+    got = step.step(0.0, v)
+    assert torch.equal(got.detach(), plain)
+    assert torch.equal(torch.autograd.grad(got, v, w)[0], w)
+    with torch.no_grad():
+        assert p.fused_for(v) and not step.step(0.0, v).requires_grad
+    with torch.autograd.forward_ad.dual_level():
+        dual = step.step(0.0, torch.autograd.forward_ad.make_dual(u, w))
+        assert torch.equal(torch.autograd.forward_ad.unpack_dual(dual).tangent, w)

@@ -517,10 +517,39 @@ class MultiPhaseAllenCahn(SemiLinearODE):
         return isinstance(u, torch.Tensor) and u.dim() == 4 and self._kernel_path(u.shape[0]) and \
             self._own_rhs(MultiPhaseAllenCahn) and not _carries_derivatives(u) and self._one_launch(u)
 
+    def _fused_pays(self, u):
+        """Whether one launch takes less time than three on the shape of ``u``.
+
+        The fused kernel works on tiles of 16 x 32 points in (y, z), with three
+        warm-up planes to a chunk of x; the separate launches work on the
+        padded points and waste no tile.  Tiles that are at least 0.4 full are
+        fused always; below that the estimates (microseconds) decide: a tile
+        point costs the fused kernel more as the phases' ring of planes leaves
+        fewer blocks on a CU, and three launches and two tensor updates take
+        38 at least.  Over 800 Euler steps of 1 to 8 phases in both types
+        (MI355X) the choice was within 0.5 % of the better one in the mean;
+        the line is missed by up to 1.4 for eight phases near it.  Three phases, fused /
+        separate: float32 64^3 11 / 39, 128^3 26 / 94, 1024 x 1 x 1024 69 / 81,
+        1024 x 1024 x 1 202 / 85, 1000000 x 1 x 1 1835 / 168; float64
+        1024 x 1 x 1024 149 / 103, 1000000 x 1 x 1 4222 / 204."""
+        n, nx, ny, nz = u.shape
+        tiles = -(-ny // 16) * -(-nz // 32)
+        if ny * nz >= 0.4 * 512 * tiles:
+            return True
+        wide = u.element_size() == 8
+        blocks = min(8, 163840 // (u.element_size() * 4 * 18 * 34 * n))  # on a CU
+        chunks = max(1, min(nx, 256 * blocks // tiles))
+        fused = 5 + (1.1 + 2.0 / blocks) * (1.62 if wide else 1.0) * 1e-6 * n * 512 * tiles * (nx + 3 * chunks)
+        if self.curvature != 1.0 or not self.fast:
+            fused *= 1.2
+        apart = 10 + (11.9 if wide else 9.0) * 1e-6 * n * (nx + 2) * (ny + 2) * (nz + 2)
+        return fused <= max(38, apart)
+
     def _one_launch(self, u):
         values = [v for _, vals in self.bc if vals is not None for v in vals]
         return self._own_pad() and self._kernel_bcs() and \
-            not any(isinstance(v, torch.Tensor) for v in values) and u.shape[2] * u.shape[3] < 2 ** 31
+            not any(isinstance(v, torch.Tensor) for v in values) and u.shape[2] * u.shape[3] < 2 ** 31 and \
+            self._fused_pays(u)
 
     def launch(self, u, out, epilogue):
         euclid = getattr(self.project_to_simplex, "__func__", None) is \
@@ -538,7 +567,7 @@ class MultiPhaseAllenCahn(SemiLinearODE):
             out = torch.empty_like(phis)
             self.launch(phis, out, _lib.make_epilogue())
             return out
-        if self._kernel_path(n):  # ghost values given as fields or by another padding: pad between the kernels
+        if self._kernel_path(n):  # ghost fields, another padding or a thin grid: pad between the kernels
             dt_code = _lib.dtype_code(phis.dtype)
             stream = _lib.stream_handle(phis.device)
             proj = torch.empty_like(phis)

@@ -112,3 +112,22 @@ def test_derivatives_of_the_state_pass_through(stepper):
     with torch.autograd.forward_ad.dual_level():
         dual = step.step(0.0, torch.autograd.forward_ad.make_dual(u, w))
         assert torch.equal(torch.autograd.forward_ad.unpack_dual(dual).tangent, w)
+
+
+@pytest.mark.parametrize("precision", ["float32", "float64"])
+@pytest.mark.parametrize("n,shape,fused", [
+    (3, (1000000, 1, 1), False), (3, (1024, 1024, 1), False), (2, (1, 400000, 1), False), (8, (65536, 2, 2), False),
+    (3, (3000, 1, 2), True), (1, (7, 7, 7), True), (6, (40, 13, 16), True), (3, (2, 300, 3), True)])
+def test_thin_grids_take_the_cheaper_route(n, shape, fused, precision):
+    """Thin grids leave the fused kernel's tiles empty; both routes give the
+    same right-hand side and step on them."""
+    p = MultiPhaseAllenCahn(grid(shape, precision), bc=BC, curvature=1.0 if n == 3 else 0.5, fast=n != 2)
+    u = phases(shape, n, p.vg.precision)
+    assert p.fused_for(u) is fused
+    got = p.rhs(0.0, u), ForwardEuler(p, 0.01).step(0.0, u)
+    p._fused_pays = lambda v: not fused
+    assert p.fused_for(u) is not fused
+    # the same operations in the same order, written twice
+    tol = 8 * torch.finfo(u.dtype).eps
+    for a, b in zip(got, (p.rhs(0.0, u), ForwardEuler(p, 0.01).step(0.0, u))):
+        assert float((a - b).abs().max()) <= tol * max(1.0, float(b.abs().max()))

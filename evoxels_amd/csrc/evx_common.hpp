@@ -110,6 +110,42 @@ __device__ __forceinline__ T apply_rules(T v, const int8_t o[3], const Bc& bc) {
   return v;
 }
 
+// Planes per chunk of a streaming launch of tiles_yz tiles (all channels), on a
+// device that holds `resident` blocks at once: the chunk that minimises
+// rounds * (planes + warm), `warm` the warm-up of a chunk in planes.  A launch
+// just above a whole number of rounds pays a whole round for its tail: the
+// 300x270x350 float32 right-hand side took 81 us with 1326 blocks on 1280
+// slots, 65 us with 19 planes more evenly split (MI355X).
+//
+// Every launch asks, so only the fullest chunk count of each round is looked
+// at (of `rounds` rounds, the most chunks have the shortest planes): at most 66
+// looks.  Looking at every count took 30 to 67 us of host time a launch on
+// grids of one tile and thousands of planes, more than their kernels.
+inline int balanced_xchunk(int64_t nx, int64_t tiles_yz, int64_t resident, int warm) {
+  const int64_t many = 8 * resident / tiles_yz + 1, most = many > 65 ? many : 65;  // chunks worth looking at
+  const int64_t last = nx < most ? nx : most;
+  int best = (int)nx;
+  double best_cost = 1e300;
+  auto look = [&](int64_t chunks) {
+    const int64_t xc = (nx + chunks - 1) / chunks, used = (nx + xc - 1) / xc;
+    const double cost = (double)((tiles_yz * used + resident - 1) / resident) * (double)(xc + warm);
+    if (cost < best_cost) {
+      best_cost = cost;
+      best = (int)xc;
+    }
+  };
+  if (tiles_yz >= resident) {  // a round or more per chunk
+    for (int64_t chunks = 1; chunks <= last; ++chunks) look(chunks);
+  } else {
+    int64_t chunks = 0;
+    for (int64_t r = 1; chunks < last; ++r) {
+      chunks = r * resident / tiles_yz;
+      look(chunks < last ? chunks : last);
+    }
+  }
+  return best;
+}
+
 template <typename T>
 __device__ __forceinline__ T clip01(T v) {
   // torch.clip(c, 0, 1): min(max(v, 0), 1), NaN propagates (both

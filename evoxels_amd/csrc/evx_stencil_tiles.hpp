@@ -290,29 +290,6 @@ __host__ inline int pick_xchunk(const Dims& d, int64_t tiles_yz, int64_t target 
   return (int)xc;
 }
 
-// Planes per chunk of a streaming launch of tiles_yz tiles (all channels), on a
-// device that holds `resident` blocks at once: the chunk that minimises
-// rounds * (planes + warm), `warm` the warm-up of a chunk in planes.  A launch
-// just above a whole number of rounds pays a whole round for its tail: the
-// 300x270x350 float32 right-hand side took 81 us with 1326 blocks on 1280
-// slots, 65 us with 19 planes more evenly split (MI355X).
-__host__ inline int balanced_xchunk(int64_t nx, int64_t tiles_yz, int64_t resident, int warm) {
-  int best = (int)nx;
-  double best_cost = 1e300;
-  for (int64_t nxc = 1; nxc <= nx; ++nxc) {
-    const int64_t xc = (nx + nxc - 1) / nxc;
-    if (nxc > 1 && (nx + nxc - 2) / (nxc - 1) == xc) continue;  // the same chunk length
-    const int64_t rounds = (tiles_yz * nxc + resident - 1) / resident;
-    const double cost = (double)rounds * (double)(xc + warm);
-    if (cost < best_cost) {
-      best_cost = cost;
-      best = (int)xc;
-    }
-    if (nxc > 64 && tiles_yz * nxc > 8 * resident) break;
-  }
-  return best;
-}
-
 // Tile grid of a streaming stencil launch of about `target` blocks; returns
 // the block count (tiles over z, y, x-chunks and channels).
 template <int BY, int TZ>

@@ -252,29 +252,30 @@ size_t align_up(size_t v) { return (v + 255) & ~size_t(255); }
 
 constexpr size_t adj_lds(size_t es) { return 9 * (size_t)(AT + 2 * APAD) * es; }
 
-int ceil_div(int a, int b) { return (a + b - 1) / b; }
+int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // Equal tiles of up to AZW voxels along z (short rows cost more than the halo they
 // save: 32 wide at 16 x 128^3 280 instead of 271 us) and as many rows as the
 // block's threads hold; along x the chunk that minimises rounds of blocks times planes a block
 // marches (its chunk and the 2*AHALO planes that it shares with its neighbours).
-AdjGeo adj_geo(int32_t dtype, const Dims& d) {
-  AdjGeo a;
-  a.nx = (int)d.nx;
-  a.ny = (int)d.ny;
-  a.nz = (int)d.nz;
-  a.c = (int)d.c;
-  a.gz = ceil_div(a.nz, AZW);
-  a.zw = ceil_div(a.nz, a.gz);
-  a.gz = ceil_div(a.nz, a.zw);
-  a.gy = ceil_div(a.ny, AT / (a.zw + 2 * AHALO) - 2 * AHALO);
-  a.tw = ceil_div(a.ny, a.gy);
-  a.gy = ceil_div(a.ny, a.tw);
-  const int64_t tiles = (int64_t)a.gz * a.gy * a.c, slots = dtype == EVX_F32 ? 512 : 256;
+// In 64 bits: the workspace query answers for any extents, also those of which
+// adj_check refuses the launch.
+struct AdjTiling {
+  int64_t zw, tw, xl, gz, gy, gx;
+  int64_t per_channel() const { return gz * gy * gx; }
+};
+
+AdjTiling adj_tiling(int32_t dtype, const Dims& d) {
+  AdjTiling a;
+  a.zw = ceil_div(d.nz, ceil_div(d.nz, AZW));
+  a.gz = ceil_div(d.nz, a.zw);
+  a.tw = ceil_div(d.ny, ceil_div(d.ny, AT / (a.zw + 2 * AHALO) - 2 * AHALO));
+  a.gy = ceil_div(d.ny, a.tw);
+  const int64_t tiles = a.gz * a.gy * d.c, slots = dtype == EVX_F32 ? 512 : 256;
   int64_t best = -1;
-  for (int n = 1; n <= std::min(a.nx, 64); ++n) {
-    const int xl = ceil_div(a.nx, n), ch = ceil_div(a.nx, xl);
-    const int64_t cost = (tiles * ch + slots - 1) / slots * (xl + 2 * AHALO);
+  for (int64_t n = 1; n <= std::min(d.nx, (int64_t)64); ++n) {
+    const int64_t xl = ceil_div(d.nx, n), ch = ceil_div(d.nx, xl);
+    const int64_t cost = ceil_div(tiles * ch, slots) * (xl + 2 * AHALO);
     if (best < 0 || cost < best) {
       best = cost;
       a.xl = xl;
@@ -282,6 +283,11 @@ AdjGeo adj_geo(int32_t dtype, const Dims& d) {
     }
   }
   return a;
+}
+
+AdjGeo adj_geo(int32_t dtype, const Dims& d) {
+  const AdjTiling t = adj_tiling(dtype, d);
+  return {(int)d.nx, (int)d.ny, (int)d.nz, (int)d.c, (int)t.zw, (int)t.tw, (int)t.xl, (int)t.gz, (int)t.gy, (int)t.gx};
 }
 
 int adj_check(const Dims& d) {
@@ -313,7 +319,7 @@ int adj_launch(const void* u, const void* w, const void* base, void* grad, doubl
 
 // Workspace: the blocks' partial sums.
 size_t ch_rhs_vjp_ws_bytes(int32_t dtype, const Dims& d) {
-  return align_up((size_t)d.c * adj_geo(dtype, d).per_channel() * 3 * sizeof(double));
+  return align_up((size_t)d.c * (size_t)adj_tiling(dtype, d).per_channel() * 3 * sizeof(double));
 }
 
 // dparams += ...; grad = base + J^T w.  With u1 != NULL (semi-implicit step)

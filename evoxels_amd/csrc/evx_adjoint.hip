@@ -257,7 +257,11 @@ int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // Equal tiles of up to AZW voxels along z (short rows cost more than the halo they
 // save: 32 wide at 16 x 128^3 280 instead of 271 us) and as many rows as the
 // block's threads hold; along x the chunk that minimises rounds of blocks times planes a block
-// marches (its chunk and the 2*AHALO planes that it shares with its neighbours).
+// marches (its chunk and the 2*AHALO planes that it shares with its neighbours).  Up to 64
+// chunks, or a block on every CU: with 64, 4000 x 12 x 60 marched 63 planes
+// in 128 blocks (float32 66.4 us, float64 94.0; 42.3 and 58.4 with 256 blocks);
+// chunks for two blocks a CU on such grids are slower again (256 x 256 x 1
+// float32 25.5 us instead of 18.3; MI355X).
 // In 64 bits: the workspace query answers for any extents, also those of which
 // adj_check refuses the launch.
 struct AdjTiling {
@@ -271,17 +275,9 @@ AdjTiling adj_tiling(int32_t dtype, const Dims& d) {
   a.gz = ceil_div(d.nz, a.zw);
   a.tw = ceil_div(d.ny, ceil_div(d.ny, AT / (a.zw + 2 * AHALO) - 2 * AHALO));
   a.gy = ceil_div(d.ny, a.tw);
-  const int64_t tiles = a.gz * a.gy * d.c, slots = dtype == EVX_F32 ? 512 : 256;
-  int64_t best = -1;
-  for (int64_t n = 1; n <= std::min(d.nx, (int64_t)64); ++n) {
-    const int64_t xl = ceil_div(d.nx, n), ch = ceil_div(d.nx, xl);
-    const int64_t cost = ceil_div(tiles * ch, slots) * (xl + 2 * AHALO);
-    if (best < 0 || cost < best) {
-      best = cost;
-      a.xl = xl;
-      a.gx = ch;
-    }
-  }
+  const int64_t tiles = a.gz * a.gy * d.c;
+  a.xl = balanced_xchunk(d.nx, tiles, dtype == EVX_F32 ? 512 : 256, 2 * AHALO, std::max<int64_t>(64, 256 / tiles));
+  a.gx = ceil_div(d.nx, a.xl);
   return a;
 }
 

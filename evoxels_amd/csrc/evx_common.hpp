@@ -112,7 +112,8 @@ __device__ __forceinline__ T apply_rules(T v, const int8_t o[3], const Bc& bc) {
 
 // Planes per chunk of a streaming launch of tiles_yz tiles (all channels), on a
 // device that holds `resident` blocks at once: the chunk that minimises
-// rounds * (planes + warm), `warm` the warm-up of a chunk in planes.  A launch
+// rounds * (planes + warm), `warm` the warm-up of a chunk in planes, of up to
+// `most` chunks (0: eight rounds of blocks, 65 at least).  A launch
 // just above a whole number of rounds pays a whole round for its tail: the
 // 300x270x350 float32 right-hand side took 81 us with 1326 blocks on 1280
 // slots, 65 us with 19 planes more evenly split (MI355X).
@@ -121,17 +122,20 @@ __device__ __forceinline__ T apply_rules(T v, const int8_t o[3], const Bc& bc) {
 // at (of `rounds` rounds, the most chunks have the shortest planes): at most 66
 // looks.  Looking at every count took 30 to 67 us of host time a launch on
 // grids of one tile and thousands of planes, more than their kernels.
-inline int balanced_xchunk(int64_t nx, int64_t tiles_yz, int64_t resident, int warm) {
-  const int64_t many = 8 * resident / tiles_yz + 1, most = many > 65 ? many : 65;  // chunks worth looking at
+inline int64_t balanced_xchunk(int64_t nx, int64_t tiles_yz, int64_t resident, int warm, int64_t most = 0) {
+  if (most == 0) {
+    most = 8 * resident / tiles_yz + 1;
+    if (most < 65) most = 65;
+  }
   const int64_t last = nx < most ? nx : most;
-  int best = (int)nx;
+  int64_t best = nx;
   double best_cost = 1e300;
   auto look = [&](int64_t chunks) {
     const int64_t xc = (nx + chunks - 1) / chunks, used = (nx + xc - 1) / xc;
     const double cost = (double)((tiles_yz * used + resident - 1) / resident) * (double)(xc + warm);
     if (cost < best_cost) {
       best_cost = cost;
-      best = (int)xc;
+      best = xc;
     }
   };
   if (tiles_yz >= resident) {  // a round or more per chunk

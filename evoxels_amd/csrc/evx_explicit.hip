@@ -491,7 +491,7 @@ unsigned x_tiles(const Dims& d, int64_t channels, int64_t resident, TileGrid* tg
   tg->ntz = (int)((d.nz + X::TZ - 1) / X::TZ);
   tg->nty = (int)((d.ny + X::BY - 1) / X::BY);
   const int64_t per = (int64_t)tg->ntz * tg->nty * channels;
-  tg->xc = balanced_xchunk(d.nx, per, resident, 3);
+  tg->xc = (int)balanced_xchunk(d.nx, per, resident, 3);
   tg->nxc = (int)((d.nx + tg->xc - 1) / tg->xc);
   return (unsigned)(per * tg->nxc);
 }

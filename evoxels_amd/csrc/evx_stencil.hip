@@ -538,7 +538,8 @@ int launch_ch_periodic(const T* u, T* out, const Dims& d, const Geo<T>& g, const
   tg.nty = (int)((d.ny + BY - 1) / BY);
   const int64_t per_chunk = (int64_t)tg.ntz * tg.nty;
   tg.xc = xb >= 0 ? SLAB_XCHUNK
-                  : balanced_xchunk(d.nx, per_chunk * d.c, EVX_RESIDENT_ROUND((ch_periodic_kernel<T, TZ, PY, false>)), 4);
+                  : (int)balanced_xchunk(d.nx, per_chunk * d.c,
+                                         EVX_RESIDENT_ROUND((ch_periodic_kernel<T, TZ, PY, false>)), 4);
   tg.nxc = (int)((d.nx + tg.xc - 1) / tg.xc);
   unsigned base = 0, blocks = (unsigned)(per_chunk * tg.nxc * d.c);
   if (xb >= 0) {  // x-slab [xa, xb) of a one-channel field, at tile-chunk granularity
@@ -767,7 +768,7 @@ static int launch_mp_fused(const void* u, void* out, const Dims& d, const Bc& bc
       return XCHUNK_BLOCKS;
     return (int64_t)per * cus;
   }();
-  tg.xc = balanced_xchunk(d.nx, (int64_t)tg.ntz * tg.nty, resident, 3);
+  tg.xc = (int)balanced_xchunk(d.nx, (int64_t)tg.ntz * tg.nty, resident, 3);
   tg.nxc = (int)((d.nx + tg.xc - 1) / tg.xc);
   const unsigned blocks = (unsigned)((int64_t)tg.ntz * tg.nty * tg.nxc);
   hipLaunchKernelGGL((mp_fused_kernel<T, NPH, EXTRA>), dim3(blocks), dim3(NT), M::LDS_BYTES, s, static_cast<const T*>(u),

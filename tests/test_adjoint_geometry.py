@@ -39,3 +39,15 @@ def test_sizes_of_ordinary_extents():
             n = C.c_size_t()
             assert _lib.load().evx_ch_rhs_vjp_workspace_bytes(dtype, C.byref(g), C.byref(n)) == 0
             assert n.value % 256 == 0 and n.value > 0
+
+
+@pytest.mark.parametrize("dims", [(1, 4000, 12, 60), (1, 4000, 1, 60), (1, 65000, 2, 2)])
+def test_long_thin_grids_fill_the_card(dims):
+    """A block (with three partial sums) on each of 256 CUs, in place of a few
+    blocks that march 60 planes and more one after another."""
+    for dtype in (0, 1):
+        g = _lib.EvxGrid()
+        g.channels, g.nx, g.ny, g.nz = dims
+        n = C.c_size_t()
+        assert _lib.load().evx_ch_rhs_vjp_workspace_bytes(dtype, C.byref(g), C.byref(n)) == 0
+        assert n.value >= 250 * 3 * 8  # equal chunks of whole planes: a few blocks fewer

@@ -20,9 +20,10 @@
 //
 // One streaming kernel evaluates all of it: mu, the faces, Gmu and the output of
 // successive planes follow each other through registers and LDS, so each field
-// crosses memory once (see adj_stream).  Every block writes its partial
-// parameter sums to its own slot and a last kernel folds them in a fixed
-// order, so results are deterministic.
+// crosses memory once (adj_stream).  Thin grids, on which its tiles would be
+// mostly halo, take three kernels with mu, Gmu and a pointwise part in memory.
+// Every block writes its partial parameter sums to its own slot and a last
+// kernel folds them in a fixed order, so results are deterministic.
 #include <algorithm>
 
 #include "evx_ch_math.hpp"
@@ -220,18 +221,210 @@ __global__ __launch_bounds__(AT, sizeof(T) == 4 ? 8 : 4) void adj_stream(
   }
 }
 
+// ---------------------------------------------------------------------------
+// The same in three kernels with mu, Gmu and the pointwise part P in memory: mu;
+// Gmu, P and the parameter sums; the output with lap(Gmu).  A voxel per
+// thread and no halo, so nothing is evaluated twice: taken where adj_stream's
+// tiles and chunks would be mostly halo (adj_separate).
+// ---------------------------------------------------------------------------
+constexpr int VZ = 64, VY = 4, VT = VZ * VY;
+
+struct AdjDims {
+  int nx, ny, nz, c;
+  int gx, gy;  // blocks along z and y per plane
+};
+
+template <typename T>
+struct VoxCoef {
+  T s18, kappa, D, eps;
+};
+template <typename T>
+__device__ __forceinline__ VoxCoef<T> vox_coef(const double* chan, double eps, double D, int c) {
+  if (chan) {
+    eps = chan[2 * c];
+    D = chan[2 * c + 1];
+  }
+  return {static_cast<T>(18.0 / eps), static_cast<T>(2.0 * eps), static_cast<T>(D), static_cast<T>(eps)};
+}
+
+// Offsets of a voxel and its six periodic neighbours inside one channel.
+struct Nb7 {
+  int64_t base;  // channel offset
+  int j, xm, xp, ym, yp, zm, zp;
+  bool valid;
+  int c, blk;  // channel, block index inside the channel
+};
+
+__device__ __forceinline__ Nb7 neighbours(const AdjDims& d) {
+  Nb7 n;
+  const int z = blockIdx.x * VZ + threadIdx.x;
+  const int y = blockIdx.y * VY + threadIdx.y;
+  const int zc = blockIdx.z;  // = c * nx + x
+  const int c = zc / d.nx, x = zc - (zc / d.nx) * d.nx;
+  n.c = c;
+  n.blk = (x * d.gy + (int)blockIdx.y) * d.gx + (int)blockIdx.x;
+  n.valid = z < d.nz && y < d.ny;
+  const int zz = n.valid ? z : 0, yy = n.valid ? y : 0;
+  const int plane = d.ny * d.nz;
+  n.base = (int64_t)c * d.nx * plane;
+  n.j = (x * d.ny + yy) * d.nz + zz;
+  n.xm = n.j + (x == 0 ? (d.nx - 1) * plane : -plane);
+  n.xp = n.j + (x == d.nx - 1 ? -(d.nx - 1) * plane : plane);
+  n.ym = n.j + (yy == 0 ? (d.ny - 1) * d.nz : -d.nz);
+  n.yp = n.j + (yy == d.ny - 1 ? -(d.ny - 1) * d.nz : d.nz);
+  n.zm = n.j + (zz == 0 ? d.nz - 1 : -1);
+  n.zp = n.j + (zz == d.nz - 1 ? -(d.nz - 1) : 1);
+  return n;
+}
+
+template <typename T>
+__device__ __forceinline__ T f_hom(T c, T s18) {
+  return ((s18 * c) * (T(1) - c)) * (T(1) - T(2) * c);
+}
+
+// Deterministic block sum of NV doubles per thread; thread 0 gets the totals.
+template <int NV>
+__device__ __forceinline__ void block_sum(double (&v)[NV]) {
+  __shared__ double red[VT / 64][NV];
+#pragma unroll
+  for (int k = 0; k < NV; ++k)
+    for (int off = 32; off > 0; off >>= 1) v[k] += __shfl_down(v[k], off, 64);
+  const int tid = threadIdx.y * VZ + threadIdx.x, wid = tid >> 6;
+  if ((tid & 63) == 0)
+#pragma unroll
+    for (int k = 0; k < NV; ++k) red[wid][k] = v[k];
+  __syncthreads();
+  if (tid == 0) {
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      double s = 0.0;
+      for (int w = 0; w < VT / 64; ++w) s += red[w][k];
+      v[k] = s;
+    }
+  }
+}
+
+// mu = f(c) - kappa*lap(c), c = clip(u).
+template <typename T>
+__global__ __launch_bounds__(VT) void adj_mu_kernel(const T* __restrict__ u, T* __restrict__ mu, AdjDims d,
+                                                    Geo<T> g, const double* __restrict__ chan, double eps,
+                                                    double D) {
+  const Nb7 n = neighbours(d);
+  if (!n.valid) return;
+  const VoxCoef<T> k = vox_coef<T>(chan, eps, D, n.c);
+  const T* uc = u + n.base;
+  const T c = clip01(uc[n.j]);
+  const T lap = Ops<false>::lap7(c, clip01(uc[n.xp]), clip01(uc[n.xm]), clip01(uc[n.yp]), clip01(uc[n.ym]),
+                                 clip01(uc[n.zp]), clip01(uc[n.zm]), g);
+  mu[n.base + n.j] = f_hom(c, k.s18) - k.kappa * lap;
+}
+
+// Gmu and P = f'(c) Gmu + 1/2 sum Kf; partial parameter sums (dD, deps).
+template <typename T>
+__global__ __launch_bounds__(VT) void adj_faces_kernel(const T* __restrict__ u, const T* __restrict__ w,
+                                                       const T* __restrict__ mu, T* __restrict__ gmu,
+                                                       T* __restrict__ pw, double* __restrict__ part, AdjDims d,
+                                                       Geo<T> g, const double* __restrict__ chan, double eps,
+                                                       double D, int nblk) {
+  const Nb7 n = neighbours(d);
+  const VoxCoef<T> k = vox_coef<T>(chan, eps, D, n.c);
+  double acc[2] = {0.0, 0.0};  // dJ/dD, dJ/deps
+  if (n.valid) {
+    const T* uc = u + n.base;
+    const T* wc = w + n.base;
+    const T* mc = mu + n.base;
+    const T cj = clip01(uc[n.j]), wj = wc[n.j], mj = mc[n.j];
+    const int lo[3] = {n.xm, n.ym, n.zm}, hi[3] = {n.xp, n.yp, n.zp};
+    const T id[3] = {g.idx, g.idy, g.idz};
+    T cn[3][2];
+    T gm = T(0), ks = T(0), dd = T(0);
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      const T cl = clip01(uc[lo[a]]), ch = clip01(uc[hi[a]]);
+      cn[a][0] = cl;
+      cn[a][1] = ch;
+      // face (j-a, j)
+      T cf = T(0.5) * (cl + cj);
+      T m = cf * (T(1) - cf);
+      T gg = (mj - mc[lo[a]]) * id[a];
+      T gf = k.D * id[a] * (wc[lo[a]] - wj);
+      const T hm = gf * m;
+      ks += gf * gg * (T(1) - T(2) * cf);
+      // face (j, j+a)
+      cf = T(0.5) * (cj + ch);
+      m = cf * (T(1) - cf);
+      gg = (mc[hi[a]] - mj) * id[a];
+      const T wd = wj - wc[hi[a]];
+      gf = k.D * id[a] * wd;
+      const T hp = gf * m;
+      ks += gf * gg * (T(1) - T(2) * cf);
+      dd += (m * gg) * (id[a] * wd);
+      gm += id[a] * (hm - hp);
+    }
+    const T fp = k.s18 * ((T(1) - T(6) * cj) + T(6) * cj * cj);
+    gmu[n.base + n.j] = gm;
+    pw[n.base + n.j] = fp * gm + T(0.5) * ks;
+    const T lapc = Ops<false>::lap7(cj, cn[0][1], cn[0][0], cn[1][1], cn[1][0], cn[2][1], cn[2][0], g);
+    const T dmu_deps = -f_hom(cj, k.s18) / k.eps - T(2) * lapc;
+    acc[0] = static_cast<double>(dd);
+    acc[1] = static_cast<double>(gm) * static_cast<double>(dmu_deps);
+  }
+  block_sum<2>(acc);
+  if (threadIdx.x == 0 && threadIdx.y == 0) {
+    double* p = part + 3 * ((int64_t)n.c * nblk + n.blk);
+    p[0] = acc[0];
+    p[1] = acc[1];
+  }
+}
+
+// out = base + mask(u) * (P - kappa lap(Gmu)); with u1 != NULL also the
+// partial of sum (w - dt*base) * (u1 - u) for the prefactor gradient.
+template <typename T>
+__global__ __launch_bounds__(VT) void adj_out_kernel(const T* __restrict__ u, const T* __restrict__ gmu,
+                                                     const T* __restrict__ pw, const T* base, T* out,
+                                                     const T* __restrict__ w, const T* __restrict__ u1,
+                                                     double dt, double* __restrict__ part, AdjDims d, Geo<T> g,
+                                                     const double* __restrict__ chan, double eps, double D,
+                                                     int nblk) {
+  const Nb7 n = neighbours(d);
+  const VoxCoef<T> k = vox_coef<T>(chan, eps, D, n.c);
+  double acc[1] = {0.0};
+  if (n.valid) {
+    const T* gc = gmu + n.base;
+    const int64_t i = n.base + n.j;
+    const T uj = u[i];
+    const T lapg = Ops<false>::lap7(gc[n.j], gc[n.xp], gc[n.xm], gc[n.yp], gc[n.ym], gc[n.zp], gc[n.zm], g);
+    const T gu = (uj >= T(0) && uj <= T(1)) ? pw[i] - k.kappa * lapg : T(0);
+    const T b = base ? base[i] : T(0);
+    out[i] = b + gu;
+    if (u1) acc[0] = static_cast<double>(w[i] - static_cast<T>(dt) * b) * static_cast<double>(u1[i] - uj);
+  }
+  if (u1) {
+    block_sum<1>(acc);
+    if (threadIdx.x == 0 && threadIdx.y == 0) part[3 * ((int64_t)n.c * nblk + n.blk) + 2] = acc[0];
+  }
+}
+
 // Per channel: fold the block partials (compensated, fixed order) and add the
 // gradients to dparams = {dJ/deps, dJ/dD}.  With step the prefactor
-// term S/(dt*theta) is added as well.
-__global__ __launch_bounds__(192) void adj_final_kernel(const double* __restrict__ part, int nblk, int step,
-                                                        double* dparams, const double* __restrict__ chan,
-                                                        double eps, double D, double dt) {
-  const int c = blockIdx.x, v = threadIdx.x >> 6, lane = threadIdx.x & 63;  // a wavefront per sum
+// term S/(dt*theta) is added as well.  W wavefronts a sum.
+template <int W>
+__global__ __launch_bounds__(192 * W) void adj_final_kernel(const double* __restrict__ part, int nblk, int step,
+                                                            double* dparams, const double* __restrict__ chan,
+                                                            double eps, double D, double dt) {
+  const int c = blockIdx.x, v = threadIdx.x / (64 * W), lane = threadIdx.x % (64 * W);
+  __shared__ SumPair wsum[3 * W];
   __shared__ double tot[3];
   SumPair s{0.0, 0.0};
-  for (int b = lane; b < nblk; b += 64) s = sum_merge(s, SumPair{part[3 * ((int64_t)c * nblk + b) + v], 0.0});
+  for (int b = lane; b < nblk; b += 64 * W) s = sum_merge(s, SumPair{part[3 * ((int64_t)c * nblk + b) + v], 0.0});
   s = wave_sum(s);
-  if (lane == 0) tot[v] = s.s + s.c;
+  if ((lane & 63) == 0) wsum[threadIdx.x >> 6] = s;
+  __syncthreads();
+  if (lane == 0) {
+    s = wsum[v * W];
+    for (int w = 1; w < W; ++w) s = sum_merge(s, wsum[v * W + w]);
+    tot[v] = s.s + s.c;
+  }
   __syncthreads();
   if (threadIdx.x == 0) {
     if (chan) {
@@ -281,9 +474,31 @@ AdjTiling adj_tiling(int32_t dtype, const Dims& d) {
   return a;
 }
 
-AdjGeo adj_geo(int32_t dtype, const Dims& d) {
-  const AdjTiling t = adj_tiling(dtype, d);
+AdjGeo adj_geo(const Dims& d, const AdjTiling& t) {
   return {(int)d.nx, (int)d.ny, (int)d.nz, (int)d.c, (int)t.zw, (int)t.tw, (int)t.xl, (int)t.gz, (int)t.gy, (int)t.gx};
+}
+
+int64_t vox_blocks(const Dims& d) { return ceil_div(d.nz, VZ) * ceil_div(d.ny, VY) * d.nx; }  // a channel's
+
+// Whether the three kernels take less time than adj_stream: asked of grids of
+// up to eight planes or rows only (small thick ones are even, 64^3 float32
+// 25.7 / 25.1 us, and adj_stream has half the launches).  Estimates in
+// microseconds: a CU works its streaming blocks off one after another, 0.70 us
+// a plane and 2.8 to start in float32 (1.25 and 5 in float64), and every block
+// marches its chunk and six planes more; the three kernels take 2.3 ns a block
+// and 4 ps a voxel (2.6 and 10).  Over 614 calls of 4 thousand to 8 million
+// voxels and 1 to 16 channels, run both ways (MI355X), they choose within 0.4 %
+// of the better one in the mean, 13 % at worst.  The three win on one or two
+// planes or rows: streaming / separate, 1 x 1024^2 float32 80 / 30 us and 8
+// channels of it 529 / 115, 8 channels of 2 x 512^2 151 / 64, 16 channels of
+// 4000 x 1 x 4 float64 321 / 140; but 3 x 200^2 float32 19 / 26.
+bool adj_separate(int32_t dtype, const Dims& d, const AdjTiling& t) {
+  if ((d.nx > 8 && d.ny > 8) || ceil_div(d.ny, VY) > 65535) return false;  // the latter: the launch's grid
+  const double rounds = (double)ceil_div(t.per_channel() * d.c, 256), planes = (double)(t.xl + 2 * AHALO);
+  const double blocks = (double)vox_blocks(d) * (double)d.c, voxels = (double)d.vol() * (double)d.c;
+  const double stream = dtype == EVX_F32 ? 10 + rounds * (0.70 * planes + 2.8) : 5 + rounds * (1.25 * planes + 5);
+  const double apart = dtype == EVX_F32 ? 18 + 2.3e-3 * blocks + 4e-6 * voxels : 20 + 2.6e-3 * blocks + 1e-5 * voxels;
+  return apart < stream;
 }
 
 int adj_check(const Dims& d) {
@@ -306,16 +521,45 @@ int adj_launch(const void* u, const void* w, const void* base, void* grad, doubl
     hipLaunchKernelGGL((adj_stream<T, false>), grid, dim3(AT), adj_lds(sizeof(T)), s, ut, wt, bt,
                        static_cast<T*>(grad), vt, dt, part, a, g, chan, eps, D);
   EVX_TRY(check_launch("adj_stream"));
-  hipLaunchKernelGGL(adj_final_kernel, dim3(a.c), dim3(192), 0, s, part, a.per_channel(), u1 ? 1 : 0, dparams, chan,
+  hipLaunchKernelGGL(adj_final_kernel<1>, dim3(a.c), dim3(192), 0, s, part, a.per_channel(), u1 ? 1 : 0, dparams, chan,
                      eps, D, dt);
+  return check_launch("adj_final_kernel");
+}
+
+template <typename T>
+int adj_launch_separate(const void* u, const void* w, const void* base, void* grad, double* dparams, const Dims& d,
+                        const Geo<T>& g, double eps, double D, const double* chan, const void* u1, double dt, void* ws,
+                        hipStream_t s) {
+  const AdjDims a{(int)d.nx, (int)d.ny, (int)d.nz, (int)d.c, (int)ceil_div(d.nz, VZ), (int)ceil_div(d.ny, VY)};
+  const size_t field = align_up((size_t)d.c * d.vol() * sizeof(T));
+  char* const p = static_cast<char*>(ws);
+  T *mu = reinterpret_cast<T*>(p), *gmu = reinterpret_cast<T*>(p + field), *pw = reinterpret_cast<T*>(p + 2 * field);
+  double* const part = reinterpret_cast<double*>(p + 3 * field);
+  const int nblk = (int)vox_blocks(d);
+  const dim3 grid(a.gx, a.gy, a.nx * a.c), block(VZ, VY);
+  const T *ut = static_cast<const T*>(u), *wt = static_cast<const T*>(w), *bt = static_cast<const T*>(base),
+          *vt = static_cast<const T*>(u1);
+  hipLaunchKernelGGL(adj_mu_kernel<T>, grid, block, 0, s, ut, mu, a, g, chan, eps, D);
+  EVX_TRY(check_launch("adj_mu_kernel"));
+  hipLaunchKernelGGL(adj_faces_kernel<T>, grid, block, 0, s, ut, wt, mu, gmu, pw, part, a, g, chan, eps, D, nblk);
+  EVX_TRY(check_launch("adj_faces_kernel"));
+  hipLaunchKernelGGL(adj_out_kernel<T>, grid, block, 0, s, ut, gmu, pw, bt, static_cast<T*>(grad), wt, vt, dt, part, a,
+                     g, chan, eps, D, nblk);
+  EVX_TRY(check_launch("adj_out_kernel"));
+  hipLaunchKernelGGL(adj_final_kernel<4>, dim3(a.c), dim3(768), 0, s, part, nblk, u1 ? 1 : 0, dparams, chan, eps, D,
+                     dt);
   return check_launch("adj_final_kernel");
 }
 
 }  // namespace
 
-// Workspace: the blocks' partial sums.
+// Workspace: the blocks' partial sums, after three fields where the kernels are separate.
 size_t ch_rhs_vjp_ws_bytes(int32_t dtype, const Dims& d) {
-  return align_up((size_t)d.c * (size_t)adj_tiling(dtype, d).per_channel() * 3 * sizeof(double));
+  const AdjTiling t = adj_tiling(dtype, d);
+  if (adj_separate(dtype, d, t))
+    return 3 * align_up((size_t)d.c * d.vol() * (dtype == EVX_F32 ? 4 : 8)) +
+           align_up((size_t)d.c * (size_t)vox_blocks(d) * 3 * sizeof(double));
+  return align_up((size_t)d.c * (size_t)t.per_channel() * 3 * sizeof(double));
 }
 
 // dparams += ...; grad = base + J^T w.  With u1 != NULL (semi-implicit step)
@@ -324,14 +568,18 @@ int ch_rhs_vjp_launch(int32_t dtype, const void* u, const void* w, const void* b
                       double* dparams, const Dims& d, const double dd[3], const double dd2[3], double eps,
                       double D, const double* chan, const void* u1, double dt, void* ws, hipStream_t s) {
   EVX_TRY(adj_check(d));
-  const AdjGeo a = adj_geo(dtype, d);
-  double* part = static_cast<double*>(ws);
   evx_grid eg{d.c, d.nx, d.ny, d.nz, {dd[0], dd[1], dd[2]}, {dd2[0], dd2[1], dd2[2]}};
-  if (dtype == EVX_F32)
-    return adj_launch<float>(u, w, base, grad, dparams, a, make_geo_from<float>(eg.div_dx, eg.div_dx2), eps, D, chan,
-                             u1, dt, part, s);
-  return adj_launch<double>(u, w, base, grad, dparams, a, make_geo_from<double>(eg.div_dx, eg.div_dx2), eps, D, chan,
-                            u1, dt, part, s);
+  const Geo<float> gf = make_geo_from<float>(eg.div_dx, eg.div_dx2);
+  const Geo<double> gd = make_geo_from<double>(eg.div_dx, eg.div_dx2);
+  const AdjTiling t = adj_tiling(dtype, d);
+  if (adj_separate(dtype, d, t))
+    return dtype == EVX_F32
+               ? adj_launch_separate<float>(u, w, base, grad, dparams, d, gf, eps, D, chan, u1, dt, ws, s)
+               : adj_launch_separate<double>(u, w, base, grad, dparams, d, gd, eps, D, chan, u1, dt, ws, s);
+  const AdjGeo a = adj_geo(d, t);
+  double* part = static_cast<double*>(ws);
+  return dtype == EVX_F32 ? adj_launch<float>(u, w, base, grad, dparams, a, gf, eps, D, chan, u1, dt, part, s)
+                          : adj_launch<double>(u, w, base, grad, dparams, a, gd, eps, D, chan, u1, dt, part, s);
 }
 
 }  // namespace evx

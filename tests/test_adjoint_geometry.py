@@ -51,3 +51,24 @@ def test_long_thin_grids_fill_the_card(dims):
         n = C.c_size_t()
         assert _lib.load().evx_ch_rhs_vjp_workspace_bytes(dtype, C.byref(g), C.byref(n)) == 0
         assert n.value >= 250 * 3 * 8  # equal chunks of whole planes: a few blocks fewer
+
+
+def query(dtype, dims):
+    g = _lib.EvxGrid()
+    g.channels, g.nx, g.ny, g.nz = dims
+    n = C.c_size_t()
+    assert _lib.load().evx_ch_rhs_vjp_workspace_bytes(dtype, C.byref(g), C.byref(n)) == 0
+    return n.value
+
+
+@pytest.mark.parametrize("dims,separate", [
+    ((1, 1, 1024, 1024), True), ((8, 2, 512, 512), True), ((16, 4000, 1, 4), True), ((4, 1024, 1, 1024), True),
+    ((1, 1, 64, 64), False), ((1, 8, 8, 8), False), ((8, 100, 100, 100), False), ((16, 128, 128, 128), False),
+    ((1, 3, 1 << 19, 4), False)])
+def test_thin_grids_take_separate_kernels(dims, separate):
+    """Where the streaming tiles would be mostly halo, mu, Gmu and the pointwise
+    part are fields of the workspace; a grid of more block rows than a launch
+    takes stays with the streaming kernel."""
+    voxels = dims[0] * dims[1] * dims[2] * dims[3]
+    for dtype, size in ((0, 4), (1, 8)):
+        assert (query(dtype, dims) >= 3 * voxels * size) is separate

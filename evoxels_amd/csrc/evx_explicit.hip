@@ -24,19 +24,11 @@
 namespace evx {
 namespace {
 
-template <typename T>
-struct XTile {  // float32: 16 x 64 points, float64: 16 x 32
-  static constexpr int TZ = sizeof(T) == 4 ? 64 : 32, PY = sizeof(T) == 4 ? 4 : 2;
-  static constexpr int BY = NT / TZ * PY, W = TZ + 2, ROWS = BY + 2, PLANE = ROWS * W;
-  static constexpr int NPT = (PLANE + NT - 1) / NT;
-};
-
 // Loads the tile's points of one x-plane into registers and writes them to
 // LDS with clip and ghost rules applied.  The y/z part of every point is
 // resolved once: periodic axes wrap, others clamp, which is the Neumann rule.
-template <typename T, bool CLIP>
+template <typename T, bool CLIP, typename X>
 struct XLoader {
-  using X = XTile<T>;
   static constexpr int NPT = X::NPT;
   uint32_t off[NPT];  // in-plane element of the source point
   uint8_t f[NPT];     // y/z ghost flags: 4/8 = y low/high, 16/32 = z low/high
@@ -56,18 +48,7 @@ struct XLoader {
 #pragma unroll
     for (int k = 0; k < NPT; ++k) {
       const int i = tid + k * NT < X::PLANE - 1 ? tid + k * NT : X::PLANE - 1;
-      int64_t gy = y0 - 1 + i / X::W, gz = z0 - 1 + i % X::W;
-      uint8_t g = 0;
-      if (gy < 0 || gy >= d.ny) {
-        if (bc.kind[1] == EVX_BC_PERIODIC) gy = wrap_near(gy, d.ny);
-        else { g |= gy < 0 ? 4 : 8; gy = gy < 0 ? 0 : d.ny - 1; }
-      }
-      if (gz < 0 || gz >= d.nz) {
-        if (bc.kind[2] == EVX_BC_PERIODIC) gz = wrap_near(gz, d.nz);
-        else { g |= gz < 0 ? 16 : 32; gz = gz < 0 ? 0 : d.nz - 1; }
-      }
-      off[k] = (uint32_t)(gy * d.nz + gz);
-      f[k] = g;
+      off[k] = X::source(i, y0, z0, d, bc, &f[k]);
     }
   }
 
@@ -139,12 +120,12 @@ struct XLoader {
 
 // A thread's view of one plane: its column rows r0-1 .. r0+PY, and the rows
 // r0-H .. of the columns at z-1, z+1 (H = 1 with corners, 0 without).
-template <typename T, int H>
+template <typename T, int H, typename X>
 struct XView {
-  static constexpr int PY = XTile<T>::PY;
+  static constexpr int PY = X::PY;
   T c[PY + 2], m[PY + 2 * H], p[PY + 2 * H];
   __device__ __forceinline__ void read(const T* s, int at) {  // at: LDS offset of the point (r0, z)
-    constexpr int W = XTile<T>::W;
+    constexpr int W = X::W;
 #pragma unroll
     for (int j = 0; j < PY + 2; ++j) c[j] = s[at + (j - 1) * W];
 #pragma unroll
@@ -229,11 +210,12 @@ __device__ __forceinline__ void x_march(int64_t x0, int64_t x1, V& a, V& b, V& c
 // Reaction-diffusion (f == 0): r = D * laplace(pad_bc(u))
 // (problem_definition.py:226-229, fd_stencils.py:62-75)
 // ---------------------------------------------------------------------------
-template <typename T, int MODE>
+template <typename T, int MODE, bool FLAT>
 __global__ __launch_bounds__(NT) void rd_rhs_kernel(const T* __restrict__ u, T* __restrict__ out, Dims d, Bc bc,
                                                     Geo<T> g, T D, Epi ep, TileGrid tg) {
-  using X = XTile<T>;
-  using Ld = XLoader<T, false>;
+  using X = XTile<T, FLAT>;
+  using Ld = XLoader<T, false, X>;
+  using View = XView<T, 0, X>;
   constexpr int PY = X::PY, W = X::W;
   __shared__ T cs[2][X::PLANE];
   const int tid = threadIdx.x, tz = tid % X::TZ, r0 = tid / X::TZ * PY;
@@ -243,7 +225,7 @@ __global__ __launch_bounds__(NT) void rd_rhs_kernel(const T* __restrict__ u, T* 
   Ld ld;
   ld.init(o.y0, o.z0, d, bc, tid);
   const int at = (r0 + 1) * W + tz + 1;
-  XView<T, 0> va, vb, vc;
+  View va, vb, vc;
   typename Ld::Plane w;
   {  // warm-up: planes x0-1 .. x0+2 in flight together
     typename Ld::Plane a, b, c;
@@ -265,7 +247,7 @@ __global__ __launch_bounds__(NT) void rd_rhs_kernel(const T* __restrict__ u, T* 
   const int rows = gz < d.nz ? (int)(gy0 + PY <= d.ny ? PY : d.ny - gy0) : 0;  // valid rows (may be <= 0)
   XOut<T, MODE> eo = x_out<T, MODE>(ep, u, out, o.ch * d.vol() + x0 * plane);
   int s = 0;  // slot of plane x+1; the other takes plane x+2
-  auto step = [&](const XView<T, 0>& vm, const XView<T, 0>& v0, XView<T, 0>& v1, int64_t x) {
+  auto step = [&](const View& vm, const View& v0, View& v1, int64_t x) {
     T eb[PY], ea[PY];
     if constexpr (MODE >= EVX_OUT_RK4_FIRST) {
 #pragma unroll
@@ -300,11 +282,12 @@ struct GsCoef {
   T Da, Db, feed, kill;
 };
 
-template <typename T, int MODE>
+template <typename T, int MODE, bool FLAT>
 __global__ __launch_bounds__(NT) void gs_rhs_kernel(const T* __restrict__ u, T* __restrict__ out, Dims d, Bc bc,
                                                     Geo<T> g, GsCoef<T> k, Epi ep, TileGrid tg) {
-  using X = XTile<T>;
-  using Ld = XLoader<T, false>;
+  using X = XTile<T, FLAT>;
+  using Ld = XLoader<T, false, X>;
+  using View = XView<T, 0, X>;
   constexpr int PY = X::PY, W = X::W;
   __shared__ T cs[2][2][X::PLANE];
   const int tid = threadIdx.x, tz = tid % X::TZ, r0 = tid / X::TZ * PY;
@@ -314,7 +297,7 @@ __global__ __launch_bounds__(NT) void gs_rhs_kernel(const T* __restrict__ u, T* 
   ld.init(o.y0, o.z0, d, bc, tid);
   const int at = (r0 + 1) * W + tz + 1;
   struct Views {
-    XView<T, 0> v[2];
+    View v[2];
   };
   Views va, vb, vc;
   typename Ld::Plane w[2];
@@ -361,7 +344,7 @@ __global__ __launch_bounds__(NT) void gs_rhs_kernel(const T* __restrict__ u, T* 
     }
 #pragma unroll
     for (int q = 0; q < PY; ++q) {
-      const XView<T, 0>&a0 = v0.v[0], &b0 = v0.v[1];
+      const View&a0 = v0.v[0], &b0 = v0.v[1];
       const T av = a0.c[q + 1], bv = b0.c[q + 1];
       const T la = lap7(av, v1.v[0].c[q + 1], vm.v[0].c[q + 1], a0.c[q + 2], a0.c[q], a0.p[q], a0.m[q], g);
       const T lb = lap7(bv, v1.v[1].c[q + 1], vm.v[1].c[q + 1], b0.c[q + 2], b0.c[q], b0.p[q], b0.m[q], g);
@@ -401,11 +384,12 @@ struct AcCoef {
   T inv_eps;   // 1/eps where eps is a power of two (the product is then the quotient), else 0
 };
 
-template <typename T, int MODE>
+template <typename T, int MODE, bool FLAT>
 __global__ __launch_bounds__(NT) void ac_rhs_kernel(const T* __restrict__ u, T* __restrict__ out, Dims d, Bc bc,
                                                     Geo<T> g, AcCoef<T> k, Epi ep, TileGrid tg) {
-  using X = XTile<T>;
-  using Ld = XLoader<T, true>;
+  using X = XTile<T, FLAT>;
+  using Ld = XLoader<T, true, X>;
+  using View = XView<T, 1, X>;
   constexpr int PY = X::PY, W = X::W;
   __shared__ T cs[2][X::PLANE];
   const int tid = threadIdx.x, tz = tid % X::TZ, r0 = tid / X::TZ * PY;
@@ -415,7 +399,7 @@ __global__ __launch_bounds__(NT) void ac_rhs_kernel(const T* __restrict__ u, T* 
   Ld ld;
   ld.init(o.y0, o.z0, d, bc, tid);
   const int at = (r0 + 1) * W + tz + 1;
-  XView<T, 1> va, vb, vc;
+  View va, vb, vc;
   typename Ld::Plane w;
   {
     typename Ld::Plane a, b, c;
@@ -437,7 +421,7 @@ __global__ __launch_bounds__(NT) void ac_rhs_kernel(const T* __restrict__ u, T* 
   const int rows = gz < d.nz ? (int)(gy0 + PY <= d.ny ? PY : d.ny - gy0) : 0;
   XOut<T, MODE> eo = x_out<T, MODE>(ep, u, out, o.ch * d.vol() + x0 * plane);
   int s = 0;
-  auto step = [&](const XView<T, 1>& vm, const XView<T, 1>& v0, XView<T, 1>& v1, int64_t x) {
+  auto step = [&](const View& vm, const View& v0, View& v1, int64_t x) {
     T eb[PY], ea[PY];
     if constexpr (MODE != EVX_OUT_RHS) {  // EULER adds to the unclipped state
 #pragma unroll
@@ -483,20 +467,7 @@ int64_t x_resident(K kernel) {
   return (int64_t)per * cus;
 }
 
-// Tile grid of a launch over `channels` channels: chunks for whole resident
-// rounds (balanced_xchunk), the warm-up counted as three planes.
-template <typename T>
-unsigned x_tiles(const Dims& d, int64_t channels, int64_t resident, TileGrid* tg) {
-  using X = XTile<T>;
-  tg->ntz = (int)((d.nz + X::TZ - 1) / X::TZ);
-  tg->nty = (int)((d.ny + X::BY - 1) / X::BY);
-  const int64_t per = (int64_t)tg->ntz * tg->nty * channels;
-  tg->xc = (int)balanced_xchunk(d.nx, per, resident, 3);
-  tg->nxc = (int)((d.nx + tg->xc - 1) / tg->xc);
-  return (unsigned)(per * tg->nxc);
-}
-
-// Launches KERNEL<T, mode> for the epilogue's mode; the resident round is
+// Launches KERNEL<T, mode, tile> for the epilogue's mode; the resident round is
 // queried once per instance (all devices of a process are taken to be alike).
 #define EVX_X_LAUNCH(KERNEL, CHANNELS, WHAT, ...)                                                        \
   switch (ep.mode) {                                                                                     \
@@ -508,13 +479,18 @@ unsigned x_tiles(const Dims& d, int64_t channels, int64_t resident, TileGrid* tg
   }                                                                                                      \
   return check_launch(WHAT);
 #define EVX_X_CASE(KERNEL, MODE, CHANNELS, ...)                                                          \
-  case MODE: {                                                                                           \
-    static const int64_t resident = x_resident(KERNEL<T, MODE>);                                         \
-    const unsigned blocks = x_tiles<T>(d, CHANNELS, resident, &tg);                                      \
-    hipLaunchKernelGGL((KERNEL<T, MODE>), dim3(blocks), dim3(NT), 0, s, static_cast<const T*>(u),        \
-                       static_cast<T*>(out), d, bc, make_geo<T>(g), __VA_ARGS__, ep, tg);                \
-    break;                                                                                               \
-  }
+  case MODE:                                                                                             \
+    if (flat_tiles<T>(d)) {                                                                              \
+      EVX_X_ONE(KERNEL, MODE, sizeof(T) == 8, CHANNELS, __VA_ARGS__)                                     \
+    } else {                                                                                             \
+      EVX_X_ONE(KERNEL, MODE, false, CHANNELS, __VA_ARGS__)                                              \
+    }                                                                                                    \
+    break;
+#define EVX_X_ONE(KERNEL, MODE, FLAT, CHANNELS, ...)                                                     \
+  static const int64_t resident = x_resident(KERNEL<T, MODE, FLAT>);                                     \
+  const unsigned blocks = x_tiles<XTile<T, FLAT>>(d, CHANNELS, resident, &tg);                           \
+  hipLaunchKernelGGL((KERNEL<T, MODE, FLAT>), dim3(blocks), dim3(NT), 0, s, static_cast<const T*>(u),    \
+                     static_cast<T*>(out), d, bc, make_geo<T>(g), __VA_ARGS__, ep, tg);
 
 template <typename T>
 int launch_rd_t(const void* u, void* out, const Dims& d, const Bc& bc, const evx_grid* g, double D, const Epi& ep,

@@ -3,9 +3,41 @@
 // LDS, so that the spectrum crosses memory once instead of three times.
 #pragma once
 #include "evx_common.hpp"
+#include "evx_fft_engine.hpp"
+#include "evx_fft_tiles.hpp"
 #include "evx_sum.hpp"
 
 namespace evx {
+
+// Radices and values per thread of a plane's lines.
+template <int N> struct PlaneSpec;
+template <> struct PlaneSpec<32>  { using R = Rad<4, 8>;    static constexpr int E = 8; };
+template <> struct PlaneSpec<48>  { using R = Rad<12, 4>;   static constexpr int E = 12; };
+template <> struct PlaneSpec<64>  { using R = Rad<8, 8>;    static constexpr int E = 8; };
+template <> struct PlaneSpec<96>  { using R = Rad<6, 4, 4>; static constexpr int E = 12; };
+template <> struct PlaneSpec<100> { using R = Rad<10, 10>;  static constexpr int E = 10; };
+template <> struct PlaneSpec<128> { using R = Rad<16, 8>;   static constexpr int E = 16; };
+#define EVX_PLANE_SIZES(X) X(32) X(48) X(64) X(96) X(100) X(128)
+
+#define X(N)                                                                                            \
+  static_assert(rad_product(PlaneSpec<N>::R{}) == N && rad_divides<PlaneSpec<N>::E>(PlaneSpec<N>::R{}), \
+                "radix plan of size " #N);
+EVX_PLANE_SIZES(X)
+#undef X
+
+template <typename T, int N>
+struct PGeo {
+  static constexpr int E = PlaneSpec<N>::E, TPL = N / E, NH = N / 2 + 1;
+  static constexpr int LINE = N + N / 16;  // padded exchange line (line_slot)
+  // rows hold NH values, one spare column for idle threads and half an exchange line
+  static constexpr int PITCH = NH + 1 > (LINE + 1) / 2 ? NH + 1 : (LINE + 1) / 2;
+  static constexpr int ROWS = N + 2;  // two spare rows for idle threads
+  static constexpr int THREADS = (NH * TPL + 63) / 64 * 64;
+  static constexpr bool WAVE = 64 % TPL == 0;  // a pair's threads share a wavefront
+  static constexpr size_t LDS = sizeof(cpx<T>) * (N + (size_t)ROWS * PITCH);
+  static_assert(N / 2 * TPL <= THREADS && THREADS <= 1024, "one round of threads");
+};
+
 
 // Whether the steps of a grid run their z and y sweeps plane by plane: ny = nz,
 // one of the lengths whose plane fits LDS in both types (128 takes 143 of

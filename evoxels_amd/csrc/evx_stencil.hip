@@ -518,35 +518,13 @@ int launch_ch(const void* u, void* out, const Dims& d, const Bc& bc, const evx_g
   return check_launch("ch_rhs_kernel");
 }
 
-constexpr int SLAB_XCHUNK = 16;
-
-// Tile of the periodic float32 right-hand side: 16 x 64 points on large grids
-// whose z length wastes no more of a 64-wide tile than of a 32-wide one, else
-// 16 x 32 (MI355X, us, 64 / 32 wide: 512^3 265 / 305, 16 x 128^3 81 / 86,
-// 256^3 36.4 / 36.4, 200^3 30.2 / 27.1, 300x270x350 64.7 / 63.7, 32^3 9.0 / 7.0).
-// Float64 tiles are 16 x 32 (400^3 285 / 257, 4 x 96^3 26 / 22).
-inline bool ch_wide_tile(const Dims& d) {
-  return (d.nz + 63) / 64 * 2 == (d.nz + 31) / 32 && d.c * d.vol() >= (int64_t(1) << 24);
-}
-
 template <typename T, int TZ, int PY>
 int launch_ch_periodic(const T* u, T* out, const Dims& d, const Geo<T>& g, const ChCoef<T>& k, const double* chan,
                        int64_t xa, int64_t xb, hipStream_t s) {
-  constexpr int BY = ChPer<T, TZ, PY>::BY;
   TileGrid tg;
-  tg.ntz = (int)((d.nz + TZ - 1) / TZ);
-  tg.nty = (int)((d.ny + BY - 1) / BY);
-  const int64_t per_chunk = (int64_t)tg.ntz * tg.nty;
-  tg.xc = xb >= 0 ? SLAB_XCHUNK
-                  : (int)balanced_xchunk(d.nx, per_chunk * d.c,
-                                         EVX_RESIDENT_ROUND((ch_periodic_kernel<T, TZ, PY, false>)), 4);
-  tg.nxc = (int)((d.nx + tg.xc - 1) / tg.xc);
-  unsigned base = 0, blocks = (unsigned)(per_chunk * tg.nxc * d.c);
-  if (xb >= 0) {  // x-slab [xa, xb) of a one-channel field, at tile-chunk granularity
-    const int64_t ca = xa / tg.xc, cb = (xb + tg.xc - 1) / tg.xc;
-    base = (unsigned)(ca * per_chunk);
-    blocks = (unsigned)((cb - ca) * per_chunk);
-  }
+  unsigned base = 0;
+  const unsigned blocks = ch_periodic_grid<ChPer<T, TZ, PY>>(
+      d, EVX_RESIDENT_ROUND((ch_periodic_kernel<T, TZ, PY, false>)), xa, xb, &tg, &base);
   auto kernel = tg.xc <= CH_SHORT ? ch_periodic_kernel<T, TZ, PY, true> : ch_periodic_kernel<T, TZ, PY, false>;
   hipLaunchKernelGGL(kernel, dim3(blocks), dim3(NT), 0, s, u, out, d, g, k, tg, chan, base);
   return check_launch("ch_periodic_kernel");

@@ -557,6 +557,35 @@ struct ChPer {
   static_assert(NHALO <= NT, "one mu halo point per thread");
 };
 
+constexpr int SLAB_XCHUNK = 16;  // planes a chunk of slab launches
+
+// Tile of the periodic float32 right-hand side: 16 x 64 points on large grids
+// whose z length wastes no more of a 64-wide tile than of a 32-wide one, else
+// 16 x 32 (MI355X, us, 64 / 32 wide: 512^3 265 / 305, 16 x 128^3 81 / 86,
+// 256^3 36.4 / 36.4, 200^3 30.2 / 27.1, 300x270x350 64.7 / 63.7, 32^3 9.0 / 7.0).
+// Float64 tiles are 16 x 32 (400^3 285 / 257, 4 x 96^3 26 / 22).
+__host__ inline bool ch_wide_tile(const Dims& d) {
+  return (d.nz + 63) / 64 * 2 == (d.nz + 31) / 32 && d.c * d.vol() >= (int64_t(1) << 24);
+}
+
+// Tile grid of the periodic kernel with tile P over the whole field (xb < 0), or
+// over the x-slab [xa, xb) of a one-channel field at tile-chunk granularity:
+// the launch then starts at tile `base`.
+template <typename P>
+__host__ inline unsigned ch_periodic_grid(const Dims& d, int64_t resident, int64_t xa, int64_t xb, TileGrid* tg,
+                                          unsigned* base) {
+  tg->ntz = (int)((d.nz + P::TZ - 1) / P::TZ);
+  tg->nty = (int)((d.ny + P::BY - 1) / P::BY);
+  const int64_t per_chunk = (int64_t)tg->ntz * tg->nty;
+  tg->xc = xb >= 0 ? SLAB_XCHUNK : (int)balanced_xchunk(d.nx, per_chunk * d.c, resident, 4);
+  tg->nxc = (int)((d.nx + tg->xc - 1) / tg->xc);
+  *base = 0;
+  if (xb < 0) return (unsigned)(per_chunk * tg->nxc * d.c);
+  const int64_t ca = xa / tg->xc, cb = (xb + tg->xc - 1) / tg->xc;
+  *base = (unsigned)(ca * per_chunk);
+  return (unsigned)((cb - ca) * per_chunk);
+}
+
 template <typename T, int TZ, int PYT, bool SHORT>
 __device__ __forceinline__ void ch_periodic_tile(const T* __restrict__ u, T* __restrict__ out, const Dims& d,
                                                  const Geo<T>& g, ChCoef<T> k, const TileGrid& tg,

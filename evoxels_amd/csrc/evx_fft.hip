@@ -794,14 +794,13 @@ int rd_spectral_step(evx_fft_plan* p, const void* u, void* u_out, void* ws, cons
   Prefac pf = make_prefac(p, 0, (-prm->D) * prm->A, prm->dt, prm->spacing);
   pf.etd = etd;
   if (etd) pf.exact = 0;
-  const bool fused = false;
   SumRec* rec = step_recs(p, ws);
   p->sums_ws = nullptr;
   EVX_TRY(p->dtype == EVX_F32 ? spectral_update<float>(p, rhs, spec, u, u_out, pf, s, rec)
                               : spectral_update<double>(p, rhs, spec, u, u_out, pf, s, rec));
   if (rec) {
     p->sums_ws = ws;
-    p->sums_n = use_planes(p) && !fused ? p->d.nx : rec_blocks(p);
+    p->sums_n = use_planes(p) ? p->d.nx : rec_blocks(p);
   }
   return EVX_OK;
 }

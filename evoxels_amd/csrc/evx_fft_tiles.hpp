@@ -210,21 +210,8 @@ __device__ __forceinline__ float etd1_f32(int jx, int jy, int jz, const Prefac& 
   return p.dt * phi;
 }
 
-__device__ __forceinline__ float prefac_f32(int jx, int jy, int jz, const Prefac& p, float sc) {
-#pragma clang fp contract(off)
-  const int sx = jx < (p.nx + 1) / 2 ? jx : jx - p.nx;
-  const int sy = jy < (p.ny + 1) / 2 ? jy : jy - p.ny;
-  const float kx = p.twopi * (static_cast<float>(sx) * p.inv_nd[0]);
-  const float ky = p.twopi * (static_cast<float>(sy) * p.inv_nd[1]);
-  const float kz = p.twopi * (static_cast<float>(jz) * p.inv_nd[2]);
-  const float k2 = (kx * kx + ky * ky) + kz * kz;
-  const float sym = p.ch ? sc * (k2 * k2) : sc * k2;
-  const float den = 1.0f - p.dt * sym;
-  return (1.0f / den) * p.dt;
-}
-
 // The float32 multiplier of one x line (jy, jz fixed): the per-line part of
-// the k^2 sum is formed once, in the same float roundings as prefac_f32
+// the k^2 sum is formed once, in the float roundings of the reference's table
 // (k^2 = (kx*kx + ky*ky) + kz*kz).  FAST takes the hardware reciprocal (1 ulp)
 // for 1/(1 - dt*sigma): used by float32 plans, whose FFT rounding is far
 // larger; float64 plans keep the IEEE quotient, so their multiplier is the

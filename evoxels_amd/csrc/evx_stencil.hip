@@ -285,7 +285,7 @@ __global__ __launch_bounds__(NT) void mp_fused_kernel(const T* __restrict__ u, T
   const int64_t x0 = o.x0, x1 = o.x1, plane = d.ny * d.nz, vol = d.vol();
 
   // the y/z part of this thread's points of a plane, resolved once
-  PlaneLoader<T, 1, M::ROWS, W, false, true> pl;
+  PlaneLoader<T, 1, M::ROWS, W, false> pl;
   pl.init(o.y0, o.z0, d, bc, tid);
   struct Plane {
     T v[NPT][NPH];
@@ -546,8 +546,6 @@ int stencil_rhs_ch_periodic(int32_t dtype, const void* u, void* out, const Dims&
                             const double div_dx2[3], double eps, double D, const double* chan, hipStream_t s,
                             int64_t xa, int64_t xb) {
   evx_grid g{d.c, d.nx, d.ny, d.nz, {div_dx[0], div_dx[1], div_dx[2]}, {div_dx2[0], div_dx2[1], div_dx2[2]}};
-  Bc b{};
-  const Epi ep{EVX_OUT_RHS, 0.0, nullptr, nullptr, nullptr};
   if (d.ny * d.nz * (dtype == EVX_F32 ? 4 : 8) >= (int64_t(1) << 32))
     return fail(EVX_ERR_UNSUPPORTED, "a (y,z) plane of more than 4 GiB");
   if (dtype == EVX_F32) {

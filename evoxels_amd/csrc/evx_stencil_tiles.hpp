@@ -64,40 +64,6 @@ __device__ __forceinline__ void epilogue(const Epi& ep, const T* __restrict__ u,
   }
 }
 
-// As epilogue(), with the state value at i supplied by the caller (no reload).
-template <typename T>
-__device__ __forceinline__ void epilogue_v(const Epi& ep, T u_i, T* __restrict__ out, int64_t i, T r) {
-#pragma clang fp contract(off)
-  const T c = static_cast<T>(ep.coef);
-  switch (ep.mode) {
-    case EVX_OUT_RHS:
-      out[i] = r;
-      break;
-    case EVX_OUT_EULER:
-      out[i] = u_i + c * r;
-      break;
-    case EVX_OUT_RK4_FIRST: {
-      const T b = ep.base ? static_cast<const T*>(ep.base)[i] : u_i;
-      out[i] = b + c * r;
-      static_cast<T*>(ep.acc_out)[i] = r;
-      break;
-    }
-    case EVX_OUT_RK4_MID: {
-      const T b = ep.base ? static_cast<const T*>(ep.base)[i] : u_i;
-      const T a = static_cast<const T*>(ep.acc_in)[i];
-      out[i] = b + c * r;
-      static_cast<T*>(ep.acc_out)[i] = a + T(2) * r;
-      break;
-    }
-    default: {
-      const T b = ep.base ? static_cast<const T*>(ep.base)[i] : u_i;
-      const T a = static_cast<const T*>(ep.acc_in)[i];
-      out[i] = b + c * (a + r);
-      break;
-    }
-  }
-}
-
 template <typename T>
 __host__ Geo<T> make_geo(const evx_grid* g) {
   return make_geo_from<T>(g->div_dx, g->div_dx2);
@@ -108,17 +74,15 @@ __host__ Geo<T> make_geo(const evx_grid* g) {
 // loads: periodic axes wrap, non-periodic ones clamp and remember the ghost
 // rule.  fetch() then only resolves the (uniform) x index of the plane and
 // issues one load per element; commit() applies clip and the ghost rules and
-// writes the element to LDS slot tid + k*NT of the plane.  With STAG the
-// staggered_x x rules are available too: an x ghost plane is then the
-// boundary node value or the zero-flux extrapolation of the first two
-// interior planes (of the clipped field when CLIP), formed in fetch().
-template <typename T, int H, int ROWS, int W, bool CLIP, bool STAG = false>
+// writes the element to LDS slot tid + k*NT of the plane.  (The multiphase kernel
+// takes the offsets and flags of init() alone.)
+template <typename T, int H, int ROWS, int W, bool CLIP>
 struct PlaneLoader {
   static constexpr int NPT = (ROWS * W + NT - 1) / NT;
   int off[NPT];      // in-plane offset y*nz + z of the source point, -1 if unused
   uint8_t yzf[NPT];  // y/z ghost flags: 4/8 = y low/high, 16/32 = z low/high
   T v[NPT];
-  uint8_t xf;        // x ghost flag of the fetched plane: 1 = low, 2 = high, 64 = final staggered value
+  uint8_t xf;        // x ghost flag of the fetched plane: 1 = low, 2 = high
 
   __device__ __forceinline__ void init(int64_t y0, int64_t z0, const Dims& d, const Bc& bc, int tid) {
 #pragma unroll
@@ -143,39 +107,10 @@ struct PlaneLoader {
     }
   }
 
-  // staggered_x ghost plane (boundary_conditions.py:96-121), in the order
-  // of the reference's expression fac1*u1 - fac2*u2 with the factors rounded
-  // to the working precision.
-  __device__ __forceinline__ void fetch_node(const T* __restrict__ uc, bool low, const Dims& d, const Bc& bc) {
-    xf = 64;
-    if (bc.kind[0] == EVX_BC_NODE_VALUE) {
-      const T v0 = static_cast<T>(low ? bc.node_lo : bc.node_hi);
-#pragma unroll
-      for (int k = 0; k < NPT; ++k) v[k] = v0;
-      return;
-    }
-    const int64_t plane = d.ny * d.nz;
-    const T* p1 = uc + (low ? 0 : d.nx - 1) * plane;
-    const T* p2 = uc + (low ? 1 : d.nx - 2) * plane;
-    const T f1 = static_cast<T>(4.0 / 3.0), f2 = static_cast<T>(1.0 / 3.0);
-#pragma unroll
-    for (int k = 0; k < NPT; ++k) {
-      if (off[k] >= 0) {
-        T a = p1[off[k]], b = p2[off[k]];
-        if (CLIP) {
-          a = clip01(a);
-          b = clip01(b);
-        }
-        v[k] = f1 * a - f2 * b;
-      }
-    }
-  }
-
   __device__ __forceinline__ void fetch(const T* __restrict__ uc, int64_t xg, const Dims& d, const Bc& bc) {
     xf = 0;
     if (xg < 0 || xg >= d.nx) {
       if (bc.kind[0] == EVX_BC_PERIODIC) xg = wrap_near(xg, d.nx);
-      else if (STAG && staggered_x(bc)) { fetch_node(uc, xg < 0, d, bc); return; }
       else { xf = xg < 0 ? 1 : 2; xg = xg < 0 ? 0 : d.nx - 1; }
     }
     const T* pl = uc + xg * (d.ny * d.nz);
@@ -188,10 +123,6 @@ struct PlaneLoader {
 #pragma unroll
     for (int k = 0; k < NPT; ++k) {
       if (off[k] >= 0) {
-        if (STAG && (xf & 64)) {
-          flat[tid + k * NT] = v[k];
-          continue;
-        }
         T x = CLIP ? clip01(v[k]) : v[k];
         const int f = xf | yzf[k];
         if (f) {
@@ -205,16 +136,15 @@ struct PlaneLoader {
   }
 };
 
-// Loader of the fully periodic tiles (the semi-implicit path): every
-// coordinate wraps, so there are no ghost rules.  Source points are kept as
-// 32-bit byte offsets from the plane base, which lets the loads use a scalar
-// base address plus a 32-bit vector offset (no 64-bit address arithmetic per
-// element).  Requires ny*nz*sizeof(T) < 2^32.
+// Source points of the fully periodic tiles (the semi-implicit path): every
+// coordinate wraps, so there are no ghost rules.  They are kept as 32-bit byte
+// offsets from the plane base, which lets the loads use a scalar base address
+// plus a 32-bit vector offset (no 64-bit address arithmetic per element).
+// Requires ny*nz*sizeof(T) < 2^32.
 template <typename T, int H, int ROWS, int W, bool CLIP>
 struct PeriodicLoader {
   static constexpr int NPT = (ROWS * W + NT - 1) / NT;
   uint32_t boff[NPT];
-  T v[NPT];
   bool last_ok;  // whether this thread's last element lies in the tile
 
   // Byte offset in its x-plane of the tile point this thread loads as
@@ -232,19 +162,6 @@ struct PeriodicLoader {
   }
 
   __device__ __forceinline__ bool valid(int k) const { return k < NPT - 1 || last_ok; }
-
-  __device__ __forceinline__ void fetch(const T* __restrict__ uc, int64_t xg, const Dims& d) {
-    const char* pl = reinterpret_cast<const char*>(uc + wrap_near(xg, d.nx) * (d.ny * d.nz));
-#pragma unroll
-    for (int k = 0; k < NPT; ++k)
-      if (valid(k)) v[k] = *reinterpret_cast<const T*>(pl + boff[k]);
-  }
-
-  __device__ __forceinline__ void commit(T* flat, int tid) const {
-#pragma unroll
-    for (int k = 0; k < NPT; ++k)
-      if (valid(k)) flat[tid + k * NT] = CLIP ? clip01(v[k]) : v[k];
-  }
 };
 
 // Ring slot of a plane at small relative index rel >= -3 (32-bit, constant modulus).
@@ -292,19 +209,16 @@ __host__ inline int pick_xchunk(const Dims& d, int64_t tiles_yz, int64_t target 
 
 // Tile grid of a streaming stencil launch of about `target` blocks; returns
 // the block count (tiles over z, y, x-chunks and channels).
-template <int BY, int TZ>
-__host__ inline unsigned stencil_tiles_of(const Dims& d, TileGrid* tg, int64_t target) {
-  const int64_t ty = (d.ny + BY - 1) / BY, tzn = (d.nz + TZ - 1) / TZ;
+template <typename T>
+__host__ inline unsigned stencil_tiles(const Dims& d, TileGrid* tg, int64_t target) {
+  constexpr int BY = NTY * TileCfg<T>::PY;
+  const int64_t ty = (d.ny + BY - 1) / BY, tzn = (d.nz + BZ - 1) / BZ;
   tg->xc = pick_xchunk(d, ty * tzn, target);
   const int64_t nxc = (d.nx + tg->xc - 1) / tg->xc;
   tg->ntz = (int)tzn;
   tg->nty = (int)ty;
   tg->nxc = (int)nxc;
   return (unsigned)(tzn * ty * nxc * d.c);
-}
-template <typename T>
-__host__ inline unsigned stencil_tiles(const Dims& d, TileGrid* tg, int64_t target) {
-  return stencil_tiles_of<NTY * TileCfg<T>::PY, BZ>(d, tg, target);
 }
 
 // ---------------------------------------------------------------------------

@@ -184,8 +184,12 @@ __device__ __forceinline__ XOut<T, MODE> x_out(const Epi& ep, const T* u, T* out
 
 // Walks the planes x0 .. x1-1 with the views of three successive planes.  ROT:
 // the views change roles (the loop written out three times) instead of being
-// copied; worth its registers in the light kernels only (256^3 float32
-// diffusion 34 -> 30 us, Allen-Cahn RK4 262 -> 313; MI355X).
+// copied.  That saves the copies and costs code and registers, so it is for
+// the kernels that are light enough: copied / changing roles at 256^3, us
+// (MI355X): diffusion Euler float32 24.7 / 23.9, float64 47.4 / 44.4, two species
+// Euler float64 114.9 / 113.7; but two species Euler float32 45.4 / 50.7,
+// diffusion RK4 float32 205 / 240, two species RK4 574 / 888, Allen-Cahn Euler
+// 50.0 / 52.9 and RK4 242 / 297.
 template <bool ROT, typename V, typename F>
 __device__ __forceinline__ void x_march(int64_t x0, int64_t x1, V& a, V& b, V& c, F&& step) {
   if constexpr (ROT) {
@@ -365,7 +369,7 @@ __global__ __launch_bounds__(NT) void gs_rhs_kernel(const T* __restrict__ u, T* 
     s ^= 1;
     __syncthreads();
   };
-  x_march<(MODE < EVX_OUT_RK4_FIRST)>(x0, x1, va, vb, vc, step);
+  x_march<(MODE < EVX_OUT_RK4_FIRST && sizeof(T) == 8)>(x0, x1, va, vb, vc, step);
 }
 
 // ---------------------------------------------------------------------------

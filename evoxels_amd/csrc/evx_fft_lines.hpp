@@ -151,15 +151,16 @@ constexpr size_t LINE_LDS = 80 * 1024;  // two blocks per CU
 // float64 need the registers of two wavefronts per SIMD.
 __host__ __device__ constexpr int line_max_threads(bool f64, bool big) { return f64 && big ? 512 : 1024; }
 
-// Strided sweeps: bricks of 128 bytes of adjacent lines (more for short
-// lines, so that a block has 256 threads, as long as the launch keeps a
-// thousand blocks), fewer where a brick would exceed the LDS.
 // Wavefronts per SIMD asked of the compiler: as many (up to `most`) as each
-// kernel's registers allow without spilling.
+// kernel's registers allow without spilling (but for two registers of the
+// float32 x sweep with prime radices).
 __host__ __device__ constexpr int line_min_waves(bool f64, bool big, int most = 6) {
   return big ? (f64 ? 2 : 4) : f64 && most > 5 ? 5 : most;
 }
 
+// Strided sweeps: bricks of 128 bytes of adjacent lines (more for short
+// lines, so that a block has 256 threads, as long as the launch keeps a
+// thousand blocks), fewer where a brick would exceed the LDS.
 template <typename T>
 inline LineGeom line_strided_geom(const LinePlan& P, int64_t nlines) {
   constexpr size_t el = sizeof(cpx<T>);

@@ -6,8 +6,8 @@
 // phase TPL threads transform a column.  The values a thread holds are those of
 // the register engine (E per thread), so a plane takes one round of threads.
 //
-// Bound: below about 32 MB of state a launch and a plane's latency (two plane
-// sweeps of 32^3 float32 take 6.6 us each, hardly more than empty launches), so
+// Bound: below about 32 MB of state a launch and a plane's latency (the two
+// sweeps of 32^3 float32 take 3.5 and 4.5 us, hardly more than empty launches), so
 // two launches instead of four are the gain; above it memory, where a plane
 // sweep reads and writes once (zy 55.8 us for 16 x 128^3 float32, 4.8 TB/s)
 // and the pair of sweeps it replaces twice (51.0 + 71.9).
@@ -18,6 +18,10 @@
 // sweeps from 34.6 to 27.0 us; 96 as 6*4*4 instead of 3*4*4*2 and 128 as 16*8
 // instead of 2*8*8 took 96^3 float32's step from 35 to 31.7 and
 // 128^3 float32's from 45.8 to 42.2 (MI355X).
+//
+// plane_inv of 128 points in float64 is held to 168 registers by its 9
+// wavefronts and spills 28 of them (116 bytes of scratch a lane): the state's
+// values wait in registers during the transform.
 #include "evx_fft_planes.hpp"
 
 namespace evx {

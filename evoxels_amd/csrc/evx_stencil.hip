@@ -1,11 +1,15 @@
 // Finite-difference right-hand sides with in-kernel boundary conditions.
 //
-// Every kernel streams along x through a ring of (y,z) planes staged in LDS
-// (2.5-D tiling): a block owns a BY x 64 tile of (y,z) and an x-chunk, loads
-// each x-plane of the tile (plus halo) once, and keeps the planes the stencil
-// needs resident.  Ghost values never exist in HBM: out-of-grid points are
-// resolved on load (periodic wrap, Neumann copy, Dirichlet 2v-u, applied x
-// then y then z as in boundary_conditions.py:33-59).
+// The Cahn-Hilliard right-hand sides and the one-launch multiphase one stream
+// along x (2.5-D tiling): a block owns a tile of (y,z) and an x-chunk, loads each
+// x-plane of the tile (plus halo) once, and keeps the planes the stencil needs
+// in a ring in LDS.  Tiles: with ghosts 16 x 64 points in float32 and 8 x 64 in
+// float64, periodic 16 x 32 or 16 x 64 (ch_wide_tile), multiphase 16 x 32.
+// Their ghost values never exist in HBM: out-of-grid points are resolved on
+// load (periodic wrap, Neumann copy, Dirichlet 2v-u, applied x then y then z as
+// in boundary_conditions.py:33-59).  The operators of the generic path (padding,
+// padded Laplacians, projection, padded multiphase and smoothed-boundary
+// right-hand sides) are a point per thread.
 //
 // Floating-point contraction is off in this file so that every product and
 // sum rounds where the reference's eager torch expression rounds.
@@ -211,10 +215,14 @@ __global__ void multiphase_rhs_kernel(const T* __restrict__ phis, const T* __res
 // projects every point (and ghost) once as it is written there, and applies
 // the step's epilogue to the raw state.  The three launches above (projection,
 // pad, right-hand side) move each phase six times; this one reads it once and
-// writes the result once.  Bound by vector issue and the plane chain (three
-// IEEE divisions a point in the projection).  A 3 x 128^3 float32
-// forward-Euler step on MI355X: 96 us in the three launches and torch's two
-// update kernels, 28 us in this one.
+// writes the result once.  Bound by vector issue and the plane chain (an IEEE
+// division a phase in the projection); from five float64 phases on, whose ring
+// leaves one block on a CU, by that block alone.  A forward-Euler step, three
+// launches and torch's two update kernels / this one, us (MI355X): 3 x 128^3
+// float32 94 / 26, float64 129 / 45; 5 x 128^3 141 / 49 and 213 / 111; 8 x 128^3
+// 218 / 87 and 379 / 176; 8 x 32^3 39 / 12 and 39 / 14; RK4 with the normal
+// Laplacian 6 x (192 x 180 x 100) 1345 / 972 and 2679 / 1981.  Thin grids, which leave
+// its tiles empty, take the three launches (the caller's rule).
 // ---------------------------------------------------------------------------
 template <typename T, int NPH>
 struct MpTile {

@@ -466,6 +466,13 @@ int check_common(int32_t dtype, const void* u, const void* out, const evx_grid* 
   return EVX_OK;
 }
 
+// Points of a (y,z) plane that a kernel's in-plane offsets of `bits` bits reach.
+int check_plane(const Dims& d, int bits) {
+  if (d.ny > (int64_t(1) << bits) / d.nz || d.plane() >= (int64_t(1) << bits))
+    return fail(EVX_ERR_UNSUPPORTED, "a (y,z) plane of 2^%d points or more", bits);
+  return EVX_OK;
+}
+
 int check_epi(const evx_epilogue* e, const void* u, const void* out, Epi* ep) {
   Epi x{EVX_OUT_RHS, 0.0, nullptr, nullptr, nullptr};
   if (e) {
@@ -633,6 +640,7 @@ extern "C" int evx_rd_rhs(int32_t dtype, const void* u, void* out, const evx_gri
   if (!bc) return fail(EVX_ERR_INVALID, "null bc");
   EVX_TRY(check_common(dtype, u, out, g, bc, &d, &b));
   EVX_TRY(check_epi(e, u, out, &ep));
+  EVX_TRY(check_plane(d, 32));
   hipStream_t s = static_cast<hipStream_t>(stream);
   return launch_rd(dtype, u, out, d, b, g, D, ep, s);
 }
@@ -647,6 +655,7 @@ extern "C" int evx_coupled_rd_rhs(int32_t dtype, const void* u, void* out, const
   EVX_TRY(check_common(dtype, u, out, g, bc, &d, &b));
   EVX_TRY(check_epi(e, u, out, &ep));
   if (d.c != 2) return fail(EVX_ERR_INVALID, "the two-species right-hand side needs exactly two channels");
+  EVX_TRY(check_plane(d, 32));
   hipStream_t s = static_cast<hipStream_t>(stream);
   return launch_gs(dtype, u, out, d, b, g, D_A, D_B, feed, kill, ep, s);
 }
@@ -662,6 +671,7 @@ extern "C" int evx_ch_rhs(int32_t dtype, const void* u, void* out, const evx_gri
   if (!(eps != 0.0)) return fail(EVX_ERR_INVALID, "eps must be nonzero");
   if (staggered_x(b))
     return fail(EVX_ERR_UNSUPPORTED, "the fused Cahn-Hilliard kernel implements the cell_center rules only");
+  EVX_TRY(check_plane(d, 31));
   hipStream_t s = static_cast<hipStream_t>(stream);
   return dtype == EVX_F32 ? launch_ch<float>(u, out, d, b, g, eps, D, ep, s)
                           : launch_ch<double>(u, out, d, b, g, eps, D, ep, s);
@@ -677,6 +687,7 @@ extern "C" int evx_ac_rhs(int32_t dtype, const void* u, void* out, const evx_gri
   EVX_TRY(check_common(dtype, u, out, g, bc, &d, &b));
   EVX_TRY(check_epi(e, u, out, &ep));
   if (!(eps != 0.0)) return fail(EVX_ERR_INVALID, "eps must be nonzero");
+  EVX_TRY(check_plane(d, 32));
   hipStream_t s = static_cast<hipStream_t>(stream);
   return launch_ac(dtype, u, out, d, b, g, eps, gab, M, force, curvature, ep, s);
 }
@@ -789,7 +800,7 @@ extern "C" int evx_multiphase_ac_rhs(int32_t dtype, const void* phis, void* out,
   if (d.c < 1 || d.c > MAX_PHASES)
     return fail(EVX_ERR_UNSUPPORTED, "the fused multiphase right-hand side handles 1 to %d phases", MAX_PHASES);
   if (!(eps != 0.0)) return fail(EVX_ERR_INVALID, "eps must be nonzero");
-  if (d.plane() >= (int64_t(1) << 31)) return fail(EVX_ERR_UNSUPPORTED, "a (y,z) plane of more than 2^31 points");
+  EVX_TRY(check_plane(d, 31));
   hipStream_t s = static_cast<hipStream_t>(stream);
   return dtype == EVX_F32 ? launch_mp<float>(phis, out, d, b, g, eps, gab, M, curvature, euclidean, ep, s)
                           : launch_mp<double>(phis, out, d, b, g, eps, gab, M, curvature, euclidean, ep, s);

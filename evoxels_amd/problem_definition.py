@@ -19,6 +19,7 @@ from typing import Any, Callable
 
 import numpy as np
 import torch
+import torch.autograd.forward_ad as _forward_ad
 
 from . import _lib
 from .voxelgrid import CellCenteredBCs, StaggeredXBCs, VoxelGridHip
@@ -125,15 +126,18 @@ class ODE(ABC):
         padding it calls and the grid's boundary rules are all unreplaced.  A
         kernel that forms ghosts itself must not run when the user's padding
         is another function (or was chosen for other boundary kinds)."""
-        mine, vg = vars(self), self.vg
-        rules = vg.bc
-        return "pad_bc" not in mine and type(self).pad_bc is ODE.pad_bc and \
-            mine.get("_pad_bc") is not None and mine["_pad_bc"] is mine.get("_builtin_pad") and \
-            (vg.convention == "cell_center" or mine.get("_pad_kinds") == self.bc_type) and \
-            type(rules) in (CellCenteredBCs, StaggeredXBCs) and len(vars(rules)) == 1 and \
-            not {"pad_bc", "pad_staggered_x", "pad_periodic"} & vars(vg).keys() and \
-            type(vg).pad_bc is VoxelGridHip.pad_bc and type(vg).pad_periodic is VoxelGridHip.pad_periodic and \
-            type(vg).pad_staggered_x is VoxelGridHip.pad_staggered_x
+        mine, vg = self.__dict__, self.vg
+        pad, rules, grid = mine.get("_pad_bc"), vg.bc, vg.__dict__
+        if pad is None or pad is not mine.get("_builtin_pad") or "pad_bc" in mine or type(self).pad_bc is not ODE.pad_bc:
+            return False
+        if type(rules) not in (CellCenteredBCs, StaggeredXBCs) or len(rules.__dict__) != 1:
+            return False
+        if "pad_bc" in grid or "pad_periodic" in grid or "pad_staggered_x" in grid:
+            return False
+        if type(vg) is not VoxelGridHip and any(getattr(type(vg), name) is not getattr(VoxelGridHip, name)
+                                                for name in ("pad_bc", "pad_periodic", "pad_staggered_x")):
+            return False
+        return vg.convention == "cell_center" or mine.get("_pad_kinds") == self.bc_type
 
     # ---- fused-kernel protocol used by the time steppers -----------------
     fused = False
@@ -216,8 +220,10 @@ def _is_default(fn) -> bool:
 
 def _carries_derivatives(u) -> bool:
     """Whether ``u`` is part of an autograd graph or holds a forward-mode tangent."""
-    return (u.requires_grad and torch.is_grad_enabled()) or \
-        torch.autograd.forward_ad.unpack_dual(u).tangent is not None
+    if u.requires_grad and torch.is_grad_enabled():
+        return True
+    # a dual tensor lives inside a dual level; where torch no longer shows the level, ask the tensor
+    return getattr(_forward_ad, "_current_level", 0) >= 0 and _forward_ad.unpack_dual(u).tangent is not None
 
 
 @dataclass
@@ -546,10 +552,10 @@ class MultiPhaseAllenCahn(SemiLinearODE):
         return fused <= max(38, apart)
 
     def _one_launch(self, u):
-        values = [v for _, vals in self.bc if vals is not None for v in vals]
-        return self._own_pad() and self._kernel_bcs() and \
-            not any(isinstance(v, torch.Tensor) for v in values) and u.shape[2] * u.shape[3] < 2 ** 31 and \
-            self._fused_pays(u)
+        for _, values in self.bc:
+            if values is not None and any(isinstance(v, torch.Tensor) for v in values):
+                return False
+        return u.shape[2] * u.shape[3] < 2 ** 31 and self._own_pad() and self._kernel_bcs() and self._fused_pays(u)
 
     def launch(self, u, out, epilogue):
         euclid = getattr(self.project_to_simplex, "__func__", None) is \
